@@ -169,7 +169,7 @@ def _pattern(shape, gen):
         c = torch.minimum(c, n - 1 - c)
         d2 = d2 + c.reshape([-1 if a == ax else 1 for a in range(len(shape))]) ** 2
     mask = d2 >= 16
-    start = o * (1 + 0.05 * torch.randn(shape, generator=gen, device=_DEV, dtype=torch.float64))
+    start = o * (1 + 0.01 * torch.randn(shape, generator=gen, device=_DEV, dtype=torch.float64))
     return (amp * mask).float(), mask, _radius(shape, 3.0) <= 1, start.to(torch.complex64)
 
 
