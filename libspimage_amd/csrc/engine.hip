@@ -1895,9 +1895,16 @@ int Engine::alloc_all() {
   return 0;
 }
 
+namespace {
+void forget_uploads(hipStream_t s);
+}
+
 Engine::~Engine() {
   // teardown: errors here have nowhere to go
-  if (s) (void)hipStreamSynchronize(s);
+  if (s) {
+    (void)hipStreamSynchronize(s);
+    forget_uploads(s);
+  }
   drop_graphs();
   void* ptrs[] = {g[0], g[1], W,        Wf,  gp,   S1,   ampx,    amp_min,  amp_max,   absb,
                   phased, flags, partials, red, hist, ctl, alg_rec, beta_rec, rec_active, Sany, Wt, ampt};
@@ -1928,10 +1935,13 @@ struct UploadRing {
   std::mutex mu;
   uint8_t* base = nullptr;
   size_t head = 0;
-  // an event is recorded on streams of the device it was created on
+  // an event is recorded on streams of the device it was created on; the
+  // runtime keeps the stream of its last record inside it, so events go with
+  // that stream (forget_uploads)
   struct Ev {
     hipEvent_t ev;
     int dev;
+    hipStream_t last;
   };
   struct Span {
     size_t off, len;
@@ -1941,6 +1951,32 @@ struct UploadRing {
   std::vector<Ev> spare;
 };
 UploadRing g_ring;
+
+// Destroys the ring's events last recorded on stream s, which the caller has
+// synchronised and is about to destroy: a later query of such an event would
+// read the stream's freed state (seen once as hipErrorCapturedEvent).
+void forget_uploads(hipStream_t s) {
+  UploadRing& g = g_ring;
+  std::lock_guard<std::mutex> lock(g.mu);
+  for (size_t i = 0; i < g.live.size();) {
+    if (g.live[i].ev.last == s) {
+      (void)hipEventDestroy(g.live[i].ev.ev);
+      g.live[i] = g.live.back();
+      g.live.pop_back();
+    } else {
+      ++i;
+    }
+  }
+  for (size_t i = 0; i < g.spare.size();) {
+    if (g.spare[i].last == s) {
+      (void)hipEventDestroy(g.spare[i].ev);
+      g.spare[i] = g.spare.back();
+      g.spare.pop_back();
+    } else {
+      ++i;
+    }
+  }
+}
 }  // namespace
 
 int upload_h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
@@ -1979,7 +2015,7 @@ int upload_h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
       ++i;
     }
   }
-  UploadRing::Ev ev{nullptr, dev};
+  UploadRing::Ev ev{nullptr, dev, s};
   for (size_t i = 0; i < g.spare.size(); ++i)
     if (g.spare[i].dev == dev) {
       ev = g.spare[i];
@@ -1988,6 +2024,7 @@ int upload_h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
       break;
     }
   if (!ev.ev) SPX_HIP(hipEventCreateWithFlags(&ev.ev, hipEventDisableTiming));
+  ev.last = s;
   memcpy(g.base + off, src, bytes);
   const hipError_t e1 = hipMemcpyAsync(dst, g.base + off, bytes, hipMemcpyHostToDevice, s);
   const hipError_t e2 = e1 == hipSuccess ? hipEventRecord(ev.ev, s) : e1;

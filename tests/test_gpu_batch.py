@@ -394,3 +394,23 @@ def test_uploads_through_a_wrapped_ring(sp):
         out.append(b.model())
         b.close()
     assert np.array_equal(out[0], out[1])
+
+
+def test_uploads_after_other_batches_streams_are_gone(sp):
+    """The upload ring outlives every batch's stream: uploads of later batches,
+    which look over the earlier uploads, still succeed and land."""
+    import gc
+    rng = np.random.default_rng(3)
+    for k in range(40):
+        b = sp.Batch((32, 32), 2)
+        a = rng.random((2, 32, 32)).astype(np.float32)
+        b.set_data(-1, a, np.ones_like(a, np.int32), (a > 0.5).astype(np.float32))
+        if k % 3:
+            b.set_support(1, a[0] > 0.25)
+        got = b.support()
+        want = a > 0.5
+        if k % 3:
+            want[1] = a[0] > 0.25
+        assert np.array_equal(got != 0, want)
+        b.close()
+        gc.collect()
