@@ -181,9 +181,6 @@ class Engine {
 
   unsigned flags_version = 0;  // bumped whenever the support bits change
   uint64_t seed = 0x5EED5EEDull;
-  // an axis has no Stockham plan: single reconstructions only, iterations
-  // unfused over Bluestein transforms (engine.hip, "Transforms of any axis length")
-  bool any_mode = false;
 
  private:
   Engine() = default;
@@ -193,10 +190,6 @@ class Engine {
   int ensure_Rf(float gamma1);
   int reduce_per_rec(int parts_per_rec, int nv, double* host_out, int count = -1);
   int blur_to_abs(float sigma, bool hist);
-  // the full transform of one or all reconstructions (shp: sh or one)
-  int fft_full(const Shape& shp, const float2* in, float2* out, int dir);
-  int iterate_any(const IterParams& p, const float* betas, int n, bool want_gp, hipEvent_t* marks);
-  float2* Sany = nullptr;  // Bluestein scratch of the any-length mode
   // the transposed Fourier-space pass (sh.tr): Wt and the amplitudes in
   // its layout, refreshed when the amplitudes change
   int ensure_transposed();
@@ -240,10 +233,9 @@ int fft_host(const float2* in, float2* out, int nx, int ny, int nz, int dir);
 int blur_host(const float2* in, float2* out, int nx, int ny, int nz, float sigma);
 // transform of device data on the library's stream (synchronous)
 int fft_device(const float2* in, float2* out, int nx, int ny, int nz, int dir);
-// The one-shot and device transforms accept any axis length up to
-// kBluesteinMaxL besides the Stockham lengths (Bluestein's method over a
-// power-of-two Stockham transform of length <= 8192); single phasers run
-// such shapes with unfused iterations, batches need Stockham lengths.
+// The one-shot and device transforms and single phasers accept any axis
+// length up to kBluesteinMaxL besides the Stockham lengths (anylen.h);
+// batches need Stockham lengths.
 constexpr int kBluesteinMaxL = 4096;
 bool fft_length_supported(int L);
 // fft_host staged through a fixed device array instead of an allocation:

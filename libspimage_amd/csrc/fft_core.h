@@ -132,7 +132,11 @@ constexpr bool mixed_plan(int L, int E, FftPlan& p) {
 // L's power-of-two part is too small for edges of E (a line of 2^a 3^b 5^c
 // 7^d with 2^a < E^2), the plan of mixed radices with edges closest to E
 // replaces it if it has fewer stages: 1000 = 2 2 5 5 5 2 becomes 10 10 10.
-constexpr FftPlan make_plan(int L, int E) {
+// E + kHalfThreads is the plan of E with half the threads, each holding twice
+// the elements.
+constexpr int kHalfThreads = 32;
+constexpr FftPlan make_plan(int L, int EH) {
+  const int E = EH % kHalfThreads;
   FftPlan p{};
   p.L = L;
   p.n = 0;
@@ -183,6 +187,7 @@ constexpr FftPlan make_plan(int L, int E) {
   p.maxr = mr;
   const int e0 = p.r[0], el = p.r[p.n - 1];
   p.T = L / (e0 / gcd_c(e0, el) * el);
+  if (EH != E) p.T /= 2;
   if (ns != L) p.ok = false;
   return p;
 }

@@ -278,6 +278,43 @@ struct SupportConstraints {
   }
 };
 
+// Gaussian transfer function of sp_gaussian_blur (src/image_filter.c:80-91)
+// with dist_to_top_left (src/image_util.c:1012-1032) at index idx of the
+// reconstruction-stacked array, computed in double and rounded to float like
+// the reference.
+__device__ __forceinline__ float blur_transfer(const ColArgs& a, long idx) {
+  const double NN = (double)((float)((long)a.nx * a.ny * a.nz));
+  const double k0 = -2.0 * (3.14159265358979323846 * 3.14159265358979323846);
+  const double s2 = (double)a.sigma * (double)a.sigma;
+  const int ix = (int)(idx % a.nx);
+  const long rest = idx / a.nx;
+  const int iy = (int)(rest % a.ny);
+  const int iz = (int)((rest / a.ny) % a.nz);  // reconstructions stack along z
+  const float dx = (a.nx - ix < ix) ? (float)(a.nx - ix) : (float)ix;
+  const float dy = (a.ny - iy < iy) ? (float)(a.ny - iy) : (float)iy;
+  const float dz = (a.nz - iz < iz) ? (float)(a.nz - iz) : (float)iz;
+  const float dist = (float)sqrt((double)dx * dx + (double)dy * dy + (double)dz * dz);
+  const float r = dist / (float)a.nx;
+  return (float)(exp(k0 * ((double)r * (double)r) * s2) / NN);
+}
+
+// One pixel's terms of the E_F sums (src/phasing.c:879-888): measured pixels
+// add (|F|-|amp|)^2 and amp^2, unmeasured ones |F|^2; FcFo sums |amp| and |F|
+// over measured pixels.  acc: nom, den, fcfo_num, fcfo_den.
+__device__ __forceinline__ void efourier_add(float2 F, float amp, double (&acc)[4]) {
+  const float af = cabsf_ref(F);
+  if (__float_as_uint(amp) != kUnmeasuredBits) {
+    const double aa = fabs((double)amp);
+    const double d = (double)af - aa;
+    acc[0] += d * d;
+    acc[1] += aa * aa;
+    acc[2] += aa;
+    acc[3] += (double)af;
+  } else {
+    acc[1] += (double)af * (double)af;
+  }
+}
+
 // Block-wide sum of NV doubles; result valid in thread 0.
 template <int NV, int NT>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double* scratch /* NV*32 */) {
@@ -322,6 +359,58 @@ struct RowShape {
   static constexpr int NT = T * M;
 };
 
+// The end of kRowBlurOut: |v[q]| stored at absb[pos(q)] where valid(q), with
+// the reconstruction's level-1 histogram (hsh: 2048 zeroed LDS counters, the
+// zeroing not yet synchronised) or running maximum.  M lines per work-group.
+template <int M, int NT, int NR, class Pos, class Valid>
+__device__ __forceinline__ void blur_out(const RowArgs& a, const float2 (&v)[NR], int blk, int line, bool act, unsigned* hsh,
+                                         float* wmax, Pos pos, Valid valid) {
+  const int tid = threadIdx.x;
+  // the work-group's lines belong to one reconstruction unless lines of
+  // several small reconstructions share it; then counts go straight to
+  // global memory
+  const int rec = line / a.lines_per_rec;
+  const int rec_first = (blk * M) / a.lines_per_rec;
+  const int last_line = (blk * M + M - 1) < a.nlines ? (blk * M + M - 1) : (a.nlines - 1);
+  const bool one_rec = rec_first == last_line / a.lines_per_rec;
+  const int slice = blockIdx.x & (kHistSlices - 1);
+  float mx = 0.f;
+  if (a.hist) __syncthreads();  // histogram zeroing done
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    if (act && valid(q)) {
+      const float m = cabsf_ref(v[q]);
+      a.absb[pos(q)] = m;
+      mx = fmaxf(mx, m);
+      if (a.hist) {
+        if (one_rec) atomicAdd(&hsh[__float_as_uint(m) >> 21], 1u);
+        else atomicAdd(&a.hist[(long)rec * kHistStride + slice * 2048 + (__float_as_uint(m) >> 21)], 1u);
+      }
+    }
+  }
+  if (a.ctl) {
+    // one atomic per work-group, into its XCD's slot
+    if (one_rec) {
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+      if ((tid & 63) == 0) wmax[tid >> 6] = mx;
+      __syncthreads();
+      if (tid == 0) {
+        for (int w = 1; w < (NT + 63) / 64; ++w) mx = fmaxf(mx, wmax[w]);
+        atomicMax(&a.ctl[rec_first * kCtlStride + kCtlMax + slice], __float_as_uint(mx));
+      }
+    } else if (act) {
+      atomicMax(&a.ctl[rec * kCtlStride + kCtlMax + slice], __float_as_uint(mx));
+    }
+  }
+  if (a.hist && one_rec) {
+    __syncthreads();
+    unsigned* h = a.hist + (long)rec_first * kHistStride + slice * 2048;
+    for (int i = tid; i < 2048; i += NT)
+      if (hsh[i]) atomicAdd(&h[i], hsh[i]);
+  }
+}
+
 template <int L, int E, int MODE>
 __global__ __launch_bounds__((RowShape<L, E>::NT)) void k_row(RowArgs a) {
   using PL = PlanOf<L, E>;
@@ -359,49 +448,8 @@ __global__ __launch_bounds__((RowShape<L, E>::NT)) void k_row(RowArgs a) {
   else fft_line<L, E, -1>(v, va, vb, t, twr);
 
   if constexpr (MODE == kRowBlurOut) {
-    // the work-group's lines belong to one reconstruction unless lines of
-    // several small reconstructions share it; then counts go straight to
-    // global memory
-    const int rec = line / a.lines_per_rec;
-    const int rec_first = (blk * M) / a.lines_per_rec;
-    const int last_line = (blk * M + M - 1) < a.nlines ? (blk * M + M - 1) : (a.nlines - 1);
-    const bool one_rec = rec_first == last_line / a.lines_per_rec;
-    const int slice = blockIdx.x & (kHistSlices - 1);
-    float mx = 0.f;
-    if (a.hist) __syncthreads();  // histogram zeroing done
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      if (act) {
-        const float m = cabsf_ref(v[q]);
-        a.absb[base + out_pos<L, E>(t, q)] = m;
-        mx = fmaxf(mx, m);
-        if (a.hist) {
-          if (one_rec) atomicAdd(&hsh[__float_as_uint(m) >> 21], 1u);
-          else atomicAdd(&a.hist[(long)rec * kHistStride + slice * 2048 + (__float_as_uint(m) >> 21)], 1u);
-        }
-      }
-    }
-    if (a.ctl) {
-      // one atomic per work-group, into its XCD's slot
-      if (one_rec) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-        if ((tid & 63) == 0) wmax[tid >> 6] = mx;
-        __syncthreads();
-        if (tid == 0) {
-          for (int w = 1; w < (NT + 63) / 64; ++w) mx = fmaxf(mx, wmax[w]);
-          atomicMax(&a.ctl[rec_first * kCtlStride + kCtlMax + slice], __float_as_uint(mx));
-        }
-      } else if (act) {
-        atomicMax(&a.ctl[rec * kCtlStride + kCtlMax + slice], __float_as_uint(mx));
-      }
-    }
-    if (a.hist && one_rec) {
-      __syncthreads();
-      unsigned* h = a.hist + (long)rec_first * kHistStride + slice * 2048;
-      for (int i = tid; i < 2048; i += NT)
-        if (hsh[i]) atomicAdd(&h[i], hsh[i]);
-    }
+    blur_out<M, NT>(a, v, blk, line, act, hsh, wmax, [&](int q) { return base + out_pos<L, E>(t, q); },
+                    [](int) { return true; });
   } else {
 #pragma unroll
     for (int q = 0; q < NR; ++q)
@@ -873,34 +921,16 @@ __global__ __launch_bounds__((ColShape<L, E, WIDE>::NT)) void k_col(ColArgs a) {
     __syncthreads();
     fft_line<L, E, +1>(v, va, vb, t, twr);
   } else if constexpr (MODE == kColBlur) {
-    // Gaussian transfer function of sp_gaussian_blur (src/image_filter.c:80-91)
-    // with dist_to_top_left (src/image_util.c:1012-1032), computed in double
-    // and rounded to float like the reference.
-    const double NN = (double)((float)((long)a.nx * a.ny * a.nz));
-    const double k0 = -2.0 * (3.14159265358979323846 * 3.14159265358979323846);
-    const double s2 = (double)a.sigma * (double)a.sigma;
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
       if (!act) continue;
-      const long idx = base + out_pos<L, E>(t, q) * st;
-      const int ix = (int)(idx % a.nx);
-      const long rest = idx / a.nx;
-      const int iy = (int)(rest % a.ny);
-      const int iz = (int)((rest / a.ny) % a.nz);  // reconstructions stack along z
-      const float dx = (a.nx - ix < ix) ? (float)(a.nx - ix) : (float)ix;
-      const float dy = (a.ny - iy < iy) ? (float)(a.ny - iy) : (float)iy;
-      const float dz = (a.nz - iz < iz) ? (float)(a.nz - iz) : (float)iz;
-      const float dist = (float)sqrt((double)dx * dx + (double)dy * dy + (double)dz * dz);
-      const float r = dist / (float)a.nx;
-      const float h = (float)(exp(k0 * ((double)r * (double)r) * s2) / NN);
+      const float h = blur_transfer(a, base + out_pos<L, E>(t, q) * st);
       v[q] = make_float2(v[q].x * h, v[q].y * h);
     }
     out_to_in<L, E>(v, va, t);
     __syncthreads();
     fft_line<L, E, +1>(v, va, vb, t, twr);
   } else if constexpr (MODE == kColEFourier) {
-    // src/phasing.c:879-888: measured pixels add (|F|-|amp|)^2 and amp^2,
-    // unmeasured ones |F|^2; FcFo sums |amp| and |F| over measured pixels.
     double acc[4] = {0.0, 0.0, 0.0, 0.0};  // nom, den, fcfo_num, fcfo_den
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
@@ -908,18 +938,7 @@ __global__ __launch_bounds__((ColShape<L, E, WIDE>::NT)) void k_col(ColArgs a) {
       const long idx = base + out_pos<L, E>(t, q) * st;
       const float2 F = v[q];
       if (a.fout) a.fout[idx] = F;
-      const float af = cabsf_ref(F);
-      const float ab = ampv[q];
-      if (__float_as_uint(ab) != kUnmeasuredBits) {
-        const double aa = fabs((double)ab);
-        const double d = (double)af - aa;
-        acc[0] += d * d;
-        acc[1] += aa * aa;
-        acc[2] += aa;
-        acc[3] += (double)af;
-      } else {
-        acc[1] += (double)af * (double)af;
-      }
+      efourier_add(F, ampv[q], acc);
     }
     block_sum<4, NT>(acc, red);
     // indexed by tile: the tiles of one reconstruction are contiguous
@@ -1218,11 +1237,20 @@ constexpr Variant variant() {
                  &LengthOps<L, E>::line_project};
 }
 
-// Dispatch table entry for one length: its compiled variants.
+// Passes of a line without a Stockham plan (anylen.h)
+struct AnyLine;
+void any_row(const AnyLine&, int mode, const RowArgs&, hipStream_t);
+void any_update(const AnyLine&, const UpdateArgs&, bool dm, hipStream_t);
+void any_col(const AnyLine&, int mode, const ColArgs&, hipStream_t);
+int any_col_blocks(const AnyLine&, const LineGeom&);
+
+// Dispatch table entry for one length: its compiled variants, or, for a
+// length without a Stockham plan, its chirp tables (nvar 0).
 struct LengthEntry {
   int L;
   int nvar;
   Variant var[3];
+  const AnyLine* any = nullptr;
 };
 
 // The passes of one axis of a shape: the length's entry and the variant the
@@ -1234,17 +1262,29 @@ struct AxisOps {
   explicit operator bool() const { return e != nullptr; }
   const AxisOps* operator->() const { return this; }
   const Variant& var() const { return e->var[v]; }
-  void row(int mode, const RowArgs& a, hipStream_t s) const { var().row(mode, a, s); }
-  void update(const UpdateArgs& a, bool dm, bool tiled, hipStream_t s) const { var().update(a, dm, tiled, s); }
-  void row_t4(const RowArgs& a, hipStream_t s) const { var().row_t4(a, s); }
-  void col(int mode, const ColArgs& a, hipStream_t s) const { var().col(mode, a, s); }
-  void col_project_wide(const ColArgs& a, hipStream_t s) const { var().col_project_wide(a, s); }
-  bool update_plain(const UpdateArgs& a, bool tiled, hipStream_t s) const { return var().update_plain(a, tiled, s); }
-  bool line_project(const ColArgs& a, hipStream_t s) const { return var().line_project(a, s); }
-  bool col_project_plain(const ColArgs& a, bool wide, hipStream_t s) const {
-    return var().col_project_plain(a, wide, s);
+  void row(int mode, const RowArgs& a, hipStream_t s) const {
+    if (e->any) any_row(*e->any, mode, a, s);
+    else var().row(mode, a, s);
   }
-  int col_blocks(const LineGeom& g) const { return var().col_blocks(g); }
+  void update(const UpdateArgs& a, bool dm, bool tiled, hipStream_t s) const {
+    if (e->any) any_update(*e->any, a, dm, s);
+    else var().update(a, dm, tiled, s);
+  }
+  void row_t4(const RowArgs& a, hipStream_t s) const { var().row_t4(a, s); }
+  void col(int mode, const ColArgs& a, hipStream_t s) const {
+    if (e->any) any_col(*e->any, mode, a, s);
+    else var().col(mode, a, s);
+  }
+  void col_project_wide(const ColArgs& a, hipStream_t s) const { var().col_project_wide(a, s); }
+  // the specialised passes; false where the general ones serve
+  bool update_plain(const UpdateArgs& a, bool tiled, hipStream_t s) const {
+    return !e->any && var().update_plain(a, tiled, s);
+  }
+  bool line_project(const ColArgs& a, hipStream_t s) const { return !e->any && var().line_project(a, s); }
+  bool col_project_plain(const ColArgs& a, bool wide, hipStream_t s) const {
+    return !e->any && var().col_project_plain(a, wide, s);
+  }
+  int col_blocks(const LineGeom& g) const { return e->any ? any_col_blocks(*e->any, g) : var().col_blocks(g); }
 };
 
 // Registry implemented by the instantiation units.
