@@ -17,7 +17,7 @@
 #include <vector>
 #include <utility>
 
-#include "passes.h"
+#include "volume.h"
 
 namespace spx {
 
@@ -66,6 +66,11 @@ struct Shape {
   // contiguous; gytr), made and undone by tiled transposes around it
   bool tr = false;
   LineGeom gytr;
+  // 3-D: the two-pass iterations (volume.h); W, Wf and the Fourier-space
+  // inputs are then in their layouts.  volr: row pass of nx, volc: column
+  // pass of nz; null where the passes per axis serve
+  const VolOps *volr = nullptr, *volc = nullptr;
+  const float2 *volr_tw = nullptr, *volc_tw = nullptr;
 };
 int make_shape(int nx, int ny, int nz, int nrec, Shape* sh);
 // elements per thread (4, 8 or 16; 0 for a trivial axis) of the x, y and z

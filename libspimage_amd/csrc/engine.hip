@@ -663,43 +663,49 @@ __global__ void k_fill_u32(unsigned* p, long n, unsigned v) {
   GRID_STRIDE(i, n) p[i] = v;
 }
 
+// Where the Fourier-space inputs (amplitudes, margins, phased amplitudes)
+// of element i of reconstruction-stacked arrays go: row-major, the 4-column
+// tiled layout of 2-D shapes, or the column pass's order of two-pass volumes
+struct FourierLayout {
+  int nx, ny, nz;
+  int t4;    // tiled
+  int volC;  // two-pass volumes: VolOps::C, else 0
+  __device__ __forceinline__ long operator()(long i) const {
+    if (!t4 && !volC) return i;
+    const long N = (long)nx * ny * nz;
+    const long r = i / N, j = i - r * N;
+    if (volC) return r * N + vol_amp_index(j, nx, ny, nz, volC);
+    const int y = (int)(j / nx), x = (int)(j - (long)y * nx);
+    return r * N + t4_offset(x, ny) + 4L * y;
+  }
+};
+
 // amplitudes as the projection reads them: unmeasured pixels get the NaN
 // pattern kUnmeasuredBits, measured NaNs the canonical quiet NaN
-// row-major index i of reconstruction-stacked (ny, nx) arrays -> index in
-// the 4-column tiled layout
-__device__ __forceinline__ long t4_index(long i, int nx, int ny) {
-  const long N = (long)nx * ny;
-  const long r = i / N, j = i - r * N;
-  const int y = (int)(j / nx), x = (int)(j - (long)y * nx);
-  return r * N + t4_offset(x, ny) + 4L * y;
-}
-
-// encoded amplitudes (unmeasured: kUnmeasuredBits), written row-major
-// (t4 == 0) or tiled
-__global__ void k_encode_amp(const float* amp, const uint8_t* flags, float* ampx, long n, int nx, int ny, int t4) {
+__global__ void k_encode_amp(const float* amp, const uint8_t* flags, float* ampx, long n, FourierLayout at) {
   GRID_STRIDE(i, n) {
     float a = amp[i];
     if (!(flags[i] & kMeasured)) a = __uint_as_float(kUnmeasuredBits);
     else if (isnan(a)) a = __uint_as_float(0x7FC00000u);
-    ampx[t4 ? t4_index(i, nx, ny) : i] = a;
+    ampx[at(i)] = a;
   }
 }
 
 // phased amplitudes of the SpRecoverAmplitudes objective; unmeasured pixels
 // carry kUnmeasuredBits in .x
-__global__ void k_encode_phased(const float2* ph, const uint8_t* flags, float2* out, long n, int nx, int ny, int t4) {
+__global__ void k_encode_phased(const float2* ph, const uint8_t* flags, float2* out, long n, FourierLayout at) {
   GRID_STRIDE(i, n) {
     const float2 v = (flags[i] & kMeasured) ? ph[i] : make_float2(__uint_as_float(kUnmeasuredBits), 0.f);
-    out[t4 ? t4_index(i, nx, ny) : i] = v;
+    out[at(i)] = v;
   }
 }
 
-__global__ void k_layout_f32(const float* in, float* out, long n, int nx, int ny, int t4) {
-  GRID_STRIDE(i, n) out[t4 ? t4_index(i, nx, ny) : i] = in[i];
+__global__ void k_layout_f32(const float* in, float* out, long n, FourierLayout at) {
+  GRID_STRIDE(i, n) out[at(i)] = in[i];
 }
 
-__global__ void k_untile_c64(const float2* in, float2* out, long n, int nx, int ny) {
-  GRID_STRIDE(i, n) out[i] = in[t4_index(i, nx, ny)];
+__global__ void k_untile_c64(const float2* in, float2* out, long n, FourierLayout at) {
+  GRID_STRIDE(i, n) out[i] = in[at(i)];
 }
 
 __global__ void k_scale_copy(const float2* in, float2* out, long n, float s) {
@@ -1206,6 +1212,96 @@ inline int rec_blocks(long n) {
 
 }  // namespace
 
+static FourierLayout layout_of(const Shape& sh) {
+  return FourierLayout{sh.nx, sh.ny, sh.nz, sh.t4 ? 1 : 0, sh.volc ? sh.volc->C : 0};
+}
+
+// ---------------------------------------------------------------------------
+// two-pass volumes (volume.h)
+// ---------------------------------------------------------------------------
+const VolOps* vol_ops_0(int L);
+const VolOps* vol_ops_1(int L);
+const VolOps* vol_ops_2(int L);
+const VolOps* vol_ops_3(int L);
+const VolOps* vol_ops_4(int L);
+const VolOps* vol_ops(int L) {
+  for (auto f : {vol_ops_0, vol_ops_1, vol_ops_2, vol_ops_3, vol_ops_4})
+    if (const VolOps* o = f(L)) return o;
+  return nullptr;
+}
+
+const float2* vol_table(int L) {
+  static std::mutex mu;
+  static std::map<int, float2*> tables;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = tables.find(L);
+  if (it != tables.end()) return it->second;
+  std::vector<float2> h((size_t)vol_table_size(L));
+  const VolCfg k = vol_cfg(L);
+  auto root = [](double j, double n) {
+    const double a = -2.0 * M_PI * j / n;
+    return make_float2((float)cos(a), (float)sin(a));
+  };
+  auto stage = [&](int off, int ns, int r) {
+    for (int q = 1; q < r; ++q)
+      for (int j = 0; j < ns; ++j) h[off + (q - 1) * ns + j] = root((double)j * q, (double)ns * r);
+  };
+  for (int i = 1; i < k.nline; ++i) stage(vol_line_off(L, i), vol_line_ns(L, i), k.line[i]);
+  stage(vol_yinv_off(L), k.y[0], k.y[1]);
+  stage(vol_yfwd_off(L), k.y[1], k.y[0]);
+  for (int b = 0; b < kVolB; ++b)
+    for (int c = 0; c < L / kVolB; ++c) h[vol_split_off(L) + b * (L / kVolB) + c] = root((double)b * c, (double)L);
+  float2* d = nullptr;
+  if (hipMalloc(&d, h.size() * sizeof(float2)) != hipSuccess) return nullptr;
+  if (hipMemcpy(d, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
+    (void)hipFree(d);
+    return nullptr;
+  }
+  tables[L] = d;
+  return d;
+}
+
+// The two-pass iterations serve every 3-D shape that has the instances
+// (SPX_NO_VOL=1 keeps the passes per axis, for A/B runs).
+static int choose_volume(Shape* sh) {
+  const char* off = getenv("SPX_NO_VOL");
+  if ((off && atoi(off) == 1) || sh->nx != sh->ny) return 0;
+  const VolOps *r = vol_ops(sh->nx), *c = vol_ops(sh->nz);
+  if (!r || !c || sh->nx % c->C) return 0;
+  sh->volr_tw = vol_table(sh->nx);
+  sh->volc_tw = vol_table(sh->nz);
+  if (!sh->volr_tw || !sh->volc_tw) {
+    set_error("could not set up the twiddle tables of a %d x %d x %d volume", sh->nx, sh->ny, sh->nz);
+    return -20;
+  }
+  sh->volr = r;
+  sh->volc = c;
+  return 0;
+}
+
+// the real-space pass, or with kVolFwd* the row-transformed iterate
+static void enqueue_vol_row(const Shape& sh, int mode, const UpdateArgs& u, hipStream_t s) {
+  VolRowArgs v{};
+  v.u = u;
+  v.tw = sh.volr_tw;
+  v.nz = sh.nz;
+  v.nplanes = sh.nz * sh.nrec;
+  sh.volr->row(mode, v, s);
+}
+
+// the Fourier-space pass on W (and on Wf behind it), or the E_F sums
+static void enqueue_vol_col(const Shape& sh, int mode, float2* W, float2* Wf, const ColArgs& a, hipStream_t s) {
+  VolColArgs v{};
+  v.a = a;
+  v.a.W = W;
+  v.W2 = Wf;
+  v.tw = sh.volc_tw;
+  v.nx = sh.nx;
+  v.ny = sh.ny;
+  v.nrec = sh.nrec;
+  sh.volc->col(mode, v, s);
+}
+
 // ---------------------------------------------------------------------------
 // shapes and pass sequences shared by the engine and the one-shot transforms
 // ---------------------------------------------------------------------------
@@ -1269,7 +1365,10 @@ int make_shape(int nx, int ny, int nz, int nrec, Shape* sh) {
     shape_variants[key] = ShapeVariants{{sh->ex.v, sh->ey.v, sh->ez.v}};
     if (!tuning_off()) record_shape(nx, ny, nz, shape_variants[key]);
   }
-  if (found[0] && found[1] && found[2]) sh->nt = tune_volume_hints(*sh);
+  if (found[0] && found[1] && found[2]) {
+    if (int rc = choose_volume(sh)) return rc;
+    sh->nt = tune_volume_hints(*sh);
+  }
   return 0;
 }
 
@@ -1377,8 +1476,8 @@ static void enqueue_fourier(const Shape& sh, int mode, const float2* in, float2*
 
 // Non-temporal hints for the iterates of a 3-D shape's real-space pass
 // (UpdateArgs::nt bits 2 and 3; W keeps ordinary accesses in 3-D), timed
-// over whole iterations of the shape (x pass, y forward, z projection, y
-// inverse) on scratch, per shape and class of batch size.  Streaming both
+// over whole iterations of the shape (two passes, or x pass, y forward, z
+// projection, y inverse) on scratch, per shape and class of batch size.  Streaming both
 // iterates took 256^3 from 269 to 247 us per HIO iteration and 96^3 x 32
 // from 546 to 500 us, but 64^3 x 32 from 122 to 129 us.  SPX_NT=<mask>
 // forces the iterate bits.  Caller holds tune_mu.
@@ -1429,10 +1528,12 @@ static int tune_volume_hints(const Shape& sh0) {
     const float ms = time_launches(
         s,
         [&] {
-          enqueue_fourier(sh, kColProject, w, w, ca, s, false);
+          if (sh.volr) enqueue_vol_col(sh, kColProject, w, nullptr, ca, s);
+          else enqueue_fourier(sh, kColProject, w, w, ca, s, false);
           u.gcur = ga;
           u.gnew = gb;
-          launch_update(sh.ex->var(), u, false, s);
+          if (sh.volr) enqueue_vol_row(sh, kVolUpdate, u, s);
+          else launch_update(sh.ex->var(), u, false, s);
           std::swap(ga, gb);
         },
         2, 5);
@@ -1455,6 +1556,7 @@ static int tune_volume_hints(const Shape& sh0) {
 
 // column tiles per reconstruction of the last axis (the efourier partials)
 static int last_axis_tiles_per_rec(const Shape& sh) {
+  if (sh.volc) return (sh.nx / sh.volc->C) * (sh.ny / kVolB);
   if (sh.ez) {
     LineGeom g = sh.gz;
     g.nouter = 1;  // one reconstruction
@@ -1669,7 +1771,7 @@ int Engine::alloc_all() {
   SPX_HIP(hipMemsetAsync(flags, 0, (size_t)NT, s));
   SPX_HIP(hipMemsetAsync(absb, 0, f, s));
   SPX_HIP(hipMemsetAsync(ctl, 0, sizeof(unsigned) * (size_t)kCtlStride * nrec, s));
-  hipLaunchKernelGGL(k_encode_amp, ew_grid(NT), dim3(256), 0, s, absb, flags, ampx, NT, nx, ny, sh.t4 ? 1 : 0);
+  hipLaunchKernelGGL(k_encode_amp, ew_grid(NT), dim3(256), 0, s, absb, flags, ampx, NT, layout_of(sh));
   // no wait: everything later on the stream is ordered behind these
   SPX_HIP(hipGetLastError());
   return 0;
@@ -1825,8 +1927,8 @@ int Engine::upload_amplitudes(const float* amp, const uint8_t* fl, int rec) {
   const long off = rec < 0 ? 0 : rec * N, n = rec < 0 ? NT : N;
   if (int rc = upload_h2d(absb + off, amp, sizeof(float) * n, s)) return rc;
   if (int rc = upload_h2d(flags + off, fl, (size_t)n, s)) return rc;
-  hipLaunchKernelGGL(k_encode_amp, ew_grid(n), dim3(256), 0, s, absb + off, flags + off, ampx + off, n, nx, ny,
-                     sh.t4 ? 1 : 0);
+  hipLaunchKernelGGL(k_encode_amp, ew_grid(n), dim3(256), 0, s, absb + off, flags + off, ampx + off, n,
+                     layout_of(sh));
   SPX_HIP(hipGetLastError());
   ++flags_version;
   ++amp_version;
@@ -1855,9 +1957,9 @@ int Engine::upload_margins(const float* lo, const float* hi) {
   if (!amp_max) SPX_HIP(hipMalloc(&amp_max, sizeof(float) * NT));
   // staged through the |blur| scratch into the Fourier-space layout
   SPX_HIP(hipMemcpyAsync(absb, lo, sizeof(float) * NT, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_layout_f32, ew_grid(NT), dim3(256), 0, s, absb, amp_min, NT, nx, ny, sh.t4 ? 1 : 0);
+  hipLaunchKernelGGL(k_layout_f32, ew_grid(NT), dim3(256), 0, s, absb, amp_min, NT, layout_of(sh));
   SPX_HIP(hipMemcpyAsync(absb, hi, sizeof(float) * NT, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_layout_f32, ew_grid(NT), dim3(256), 0, s, absb, amp_max, NT, nx, ny, sh.t4 ? 1 : 0);
+  hipLaunchKernelGGL(k_layout_f32, ew_grid(NT), dim3(256), 0, s, absb, amp_max, NT, layout_of(sh));
   SPX_HIP(hipGetLastError());
   SPX_HIP(hipStreamSynchronize(s));
   return 0;
@@ -1868,7 +1970,7 @@ int Engine::upload_phased(const float2* ph, const uint8_t* fl) {
   if (!phased) SPX_HIP(hipMalloc(&phased, sizeof(float2) * NT));
   SPX_HIP(hipMemcpyAsync(S1, ph, sizeof(float2) * NT, hipMemcpyHostToDevice, s));
   SPX_HIP(hipMemcpyAsync(flags, fl, (size_t)NT, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_encode_phased, ew_grid(NT), dim3(256), 0, s, S1, flags, phased, NT, nx, ny, sh.t4 ? 1 : 0);
+  hipLaunchKernelGGL(k_encode_phased, ew_grid(NT), dim3(256), 0, s, S1, flags, phased, NT, layout_of(sh));
   SPX_HIP(hipGetLastError());
   SPX_HIP(hipStreamSynchronize(s));
   ++flags_version;
@@ -2021,7 +2123,25 @@ int Engine::ensure_transposed() {
 }
 
 int Engine::ensure_R() {
-  if (!R_valid) {
+  if (sh.volr) {
+    // reconstructions in order of their slots; one call for all when none is valid
+    std::sort(R_stale.begin(), R_stale.end());
+    R_stale.erase(std::unique(R_stale.begin(), R_stale.end()), R_stale.end());
+    UpdateArgs u{};
+    if (!R_valid) {
+      u.gcur = g[cur];
+      u.W = W;
+      enqueue_vol_row(sh, kVolFwd, u, s);
+    } else {
+      for (int r : R_stale) {
+        u.gcur = g[cur] + (long)r * N;
+        u.W = W + (long)r * N;
+        enqueue_vol_row(one, kVolFwd, u, s);
+      }
+    }
+    R_valid = true;
+    R_stale.clear();
+  } else if (!R_valid) {
     if (sh.t4) sh.ex->row_t4(row_args(sh, g[cur], W), s);
     else sh.ex->row(kRowFwd, row_args(sh, g[cur], W), s);
     R_valid = true;
@@ -2044,7 +2164,14 @@ int Engine::ensure_R() {
 int Engine::ensure_Rf(float gamma1) {
   if (!Wf) SPX_HIP(hipMalloc(&Wf, sizeof(float2) * NT));
   if (Rf_valid && Rf_version == flags_version && Rf_gamma1 == gamma1) return 0;
-  if (sh.t4) {
+  if (sh.volr) {
+    UpdateArgs u{};
+    u.gcur = g[cur];
+    u.W = Wf;
+    u.flags = flags;
+    u.gamma1 = gamma1;
+    enqueue_vol_row(sh, kVolFwdF1, u, s);
+  } else if (sh.t4) {
     // the tiled transform cannot run in place: f1 goes through the scratch
     hipLaunchKernelGGL(k_dm_f1, ew_grid(NT), dim3(256), 0, s, g[cur], flags, gamma1, S1, NT);
     sh.ex->row_t4(row_args(sh, S1, Wf), s);
@@ -2106,9 +2233,13 @@ int Engine::iterate_impl(const IterParams& p, const float* betas, int n, bool wa
     if (int r = ensure_transposed()) return r;
   for (int i = 0; i < n; ++i) {
     if (marks) SPX_HIP(hipEventRecord(marks[2 * i], s));
-    if (trp) enqueue_fourier_transposed(sh, W, Wt, ampt, ca, s);
-    else enqueue_fourier(sh, kColProject, W, W, ca, s, sh.t4);
-    if (dm) enqueue_fourier(sh, kColProject, Wf, Wf, caf, s, sh.t4);
+    if (sh.volc) {
+      enqueue_vol_col(sh, kColProject, W, dm ? Wf : nullptr, ca, s);
+    } else {
+      if (trp) enqueue_fourier_transposed(sh, W, Wt, ampt, ca, s);
+      else enqueue_fourier(sh, kColProject, W, W, ca, s, sh.t4);
+      if (dm) enqueue_fourier(sh, kColProject, Wf, Wf, caf, s, sh.t4);
+    }
     if (marks) SPX_HIP(hipEventRecord(marks[2 * i + 1], s));
     u.gcur = g[cur];
     u.gnew = g[cur ^ 1];
@@ -2117,7 +2248,8 @@ int Engine::iterate_impl(const IterParams& p, const float* betas, int n, bool wa
     // the specialised pass: ER / HIO / RAAR without gp (per-reconstruction
     // tables and idle slots in its TAB form)
     const bool plain = !dm && !u.gp && !plain_off();
-    if (!(plain && sh.ex->update_plain(u, sh.t4, s))) sh.ex->update(u, dm, sh.t4, s);
+    if (sh.volr) enqueue_vol_row(sh, dm ? kVolUpdateDM : kVolUpdate, u, s);
+    else if (!(plain && sh.ex->update_plain(u, sh.t4, s))) sh.ex->update(u, dm, sh.t4, s);
     cur ^= 1;
   }
   if (marks) SPX_HIP(hipEventRecord(marks[2 * n], s));
@@ -2236,8 +2368,9 @@ int Engine::efourier(double* out, float2* fout) {
   ca.ampx = ampx;
   ca.partials = partials;
   ca.fout = fout;
-  // the 3-D path needs somewhere to put the y-transformed lines: S1
-  enqueue_fourier(sh, kColEFourier, W, S1, ca, s, sh.t4);
+  // the passes per axis need somewhere to put the y-transformed lines: S1
+  if (sh.volc) enqueue_vol_col(sh, kColEFourier, W, nullptr, ca, s);
+  else enqueue_fourier(sh, kColEFourier, W, S1, ca, s, sh.t4);
   SPX_HIP(hipGetLastError());
   return reduce_per_rec(last_axis_tiles_per_rec(sh), 4, out);
 }
@@ -2248,7 +2381,8 @@ int Engine::efourier_enqueue() {
   ColArgs ca{};
   ca.ampx = ampx;
   ca.partials = partials;
-  enqueue_fourier(sh, kColEFourier, W, S1, ca, s, sh.t4);
+  if (sh.volc) enqueue_vol_col(sh, kColEFourier, W, nullptr, ca, s);
+  else enqueue_fourier(sh, kColEFourier, W, S1, ca, s, sh.t4);
   SPX_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_reduce_rec, dim3(nrec), dim3(256), 0, s, partials, last_axis_tiles_per_rec(sh), 4, red);
   SPX_HIP(hipGetLastError());
@@ -2273,7 +2407,7 @@ int Engine::fmodel(float2* fout) {
   if (!sh.t4) return efourier(dummy.data(), fout);
   // the transform comes out in the tiled layout: untile it into `fout`
   if (int r = efourier(dummy.data(), S1)) return r;
-  hipLaunchKernelGGL(k_untile_c64, ew_grid(NT), dim3(256), 0, s, S1, fout, NT, nx, ny);
+  hipLaunchKernelGGL(k_untile_c64, ew_grid(NT), dim3(256), 0, s, S1, fout, NT, layout_of(sh));
   SPX_HIP(hipGetLastError());
   return 0;
 }

@@ -268,59 +268,121 @@ __device__ __forceinline__ void dft4(float2& x0, float2& x1, float2& x2, float2&
   x3 = csub(t1, t3);
 }
 
-template <int DIR>
+// The small DFTs multiply by the same constants in every transform, and the
+// rounded pairs are off to one side (|w_16| by -2.9e-8, |w_8| by -1.7e-8), so
+// over iterations these errors add up instead of averaging out.  With COMP
+// the constants' rounding errors are put back, one multiply-add per product:
+// after 10 forward and inverse transforms, 16 x 16 points are 8.3e-7 off
+// without and 4.5e-7 with it (8 x 4 x 8: 6.6e-7 and 5.2e-7; 12 x 16 5.9e-7 and
+// 4.7e-7).  The two-pass volumes use it (256^3 HIO, 3 iterations against
+// float64: 4.0e-7 -> 2.5e-7; +1 % time); 2-D passes, bound by their
+// instructions, do not.
+constexpr float kRtHalf = 0.70710678118654752440f;
+constexpr float kRtHalfLo = (float)(0.70710678118654752440 - (double)kRtHalf);
+// a (c + DIR i s), the constants in double
+template <int DIR, bool COMP>
+__device__ __forceinline__ float2 rotc(float2 a, double c, double s) {
+  const float ch = (float)c, sh = (float)s;
+  if constexpr (COMP) {
+    const float cl = (float)(c - (double)ch), sl = (float)(s - (double)sh);
+    return make_float2(fmaf(a.x, ch, fmaf(-DIR * a.y, sh, fmaf(a.x, cl, -DIR * a.y * sl))),
+                       fmaf(a.y, ch, fmaf(DIR * a.x, sh, fmaf(a.y, cl, DIR * a.x * sl))));
+  }
+  return make_float2(a.x * ch - DIR * a.y * sh, a.y * ch + DIR * a.x * sh);
+}
+// c a, c = hi + lo
+template <bool COMP>
+__device__ __forceinline__ float scale_c(float a, float hi, float lo) {
+  if constexpr (COMP) return fmaf(a, hi, a * lo);
+  return hi * a;
+}
+
+template <int DIR, bool COMP = false>
 __device__ __forceinline__ void dft8(float2* x) {
-  constexpr float c = 0.70710678118654752440f;
+  constexpr float c = kRtHalf, l = kRtHalfLo;
   float2 e0 = x[0], e1 = x[2], e2 = x[4], e3 = x[6];
   float2 o0 = x[1], o1 = x[3], o2 = x[5], o3 = x[7];
   dft4<DIR>(e0, e1, e2, e3);
   dft4<DIR>(o0, o1, o2, o3);
   // W8^1 = (c, DIR c), W8^2 = DIR i, W8^3 = (-c, DIR c)
-  const float2 w1 = make_float2(c * (o1.x - DIR * o1.y), c * (o1.y + DIR * o1.x));
+  const float2 w1 = make_float2(scale_c<COMP>(o1.x - DIR * o1.y, c, l), scale_c<COMP>(o1.y + DIR * o1.x, c, l));
   const float2 w2 = rot<DIR>(o2);
-  const float2 w3 = make_float2(c * (-o3.x - DIR * o3.y), c * (-o3.y + DIR * o3.x));
+  const float2 w3 = make_float2(scale_c<COMP>(-o3.x - DIR * o3.y, c, l), scale_c<COMP>(-o3.y + DIR * o3.x, c, l));
   x[0] = cadd(e0, o0); x[4] = csub(e0, o0);
   x[1] = cadd(e1, w1); x[5] = csub(e1, w1);
   x[2] = cadd(e2, w2); x[6] = csub(e2, w2);
   x[3] = cadd(e3, w3); x[7] = csub(e3, w3);
 }
 
-template <int DIR>
+template <int DIR, bool COMP = false>
 __device__ __forceinline__ void dft16(float2* x) {
   float2 e[8], o[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) { e[k] = x[2 * k]; o[k] = x[2 * k + 1]; }
-  dft8<DIR>(e);
-  dft8<DIR>(o);
+  dft8<DIR, COMP>(e);
+  dft8<DIR, COMP>(o);
   // W16^r = (cos(2 pi r/16), DIR sin(2 pi r/16))
-  constexpr float C1 = 0.92387953251128675613f, S1 = 0.38268343236508977173f;
-  constexpr float C2 = 0.70710678118654752440f;
-  const float cs[8] = {1.f, C1, C2, S1, 0.f, -S1, -C2, -C1};
-  const float sn[8] = {0.f, S1, C2, C1, 1.f, C1, C2, S1};
+  constexpr double C1 = 0.92387953251128675613, S1 = 0.38268343236508977173;
+  constexpr double C2 = 0.70710678118654752440;
+  const double cs[8] = {1., C1, C2, S1, 0., -S1, -C2, -C1};
+  const double sn[8] = {0., S1, C2, C1, 1., C1, C2, S1};
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
     float2 w;
     if (r == 0) w = o[0];
     else if (r == 4) w = rot<DIR>(o[4]);
-    else w = make_float2(o[r].x * cs[r] - DIR * o[r].y * sn[r], o[r].y * cs[r] + DIR * o[r].x * sn[r]);
+    else w = rotc<DIR, COMP>(o[r], cs[r], sn[r]);
     x[r] = cadd(e[r], w);
     x[r + 8] = csub(e[r], w);
   }
 }
 
-template <int DIR>
+template <int DIR, bool COMP = false>
 __device__ __forceinline__ void dft3(float2* x) {
   constexpr float h = 0.86602540378443864676f;  // sqrt(3)/2
+  constexpr float l = (float)(0.86602540378443864676 - (double)h);
   const float2 s = cadd(x[1], x[2]);
   const float2 d = rot<DIR>(csub(x[1], x[2]));
-  const float2 m = make_float2(x[0].x - 0.5f * s.x, x[0].y - 0.5f * s.y);
+  float2 m = make_float2(x[0].x - 0.5f * s.x, x[0].y - 0.5f * s.y);
   x[0] = cadd(x[0], s);
+  if constexpr (COMP) {
+    x[1] = make_float2(fmaf(h, d.x, fmaf(l, d.x, m.x)), fmaf(h, d.y, fmaf(l, d.y, m.y)));
+    x[2] = make_float2(fmaf(-h, d.x, fmaf(-l, d.x, m.x)), fmaf(-h, d.y, fmaf(-l, d.y, m.y)));
+    return;
+  }
   x[1] = make_float2(m.x + h * d.x, m.y + h * d.y);
   x[2] = make_float2(m.x - h * d.x, m.y - h * d.y);
 }
 
-template <int DIR>
+// a p + b q, the constants in double
+template <bool COMP>
+__device__ __forceinline__ float2 lin2(double a, float2 p, double b, float2 q) {
+  const float ah = (float)a, bh = (float)b;
+  if constexpr (COMP) {
+    const float al = (float)(a - (double)ah), bl = (float)(b - (double)bh);
+    return make_float2(fmaf(ah, p.x, fmaf(bh, q.x, fmaf(al, p.x, bl * q.x))),
+                       fmaf(ah, p.y, fmaf(bh, q.y, fmaf(al, p.y, bl * q.y))));
+  }
+  return make_float2(ah * p.x + bh * q.x, ah * p.y + bh * q.y);
+}
+
+template <int DIR, bool COMP = false>
 __device__ __forceinline__ void dft5(float2* x) {
+  if constexpr (COMP) {
+    constexpr double c1 = 0.30901699437494742410, c2 = -0.80901699437494742410;
+    constexpr double s1 = 0.95105651629515357212, s2 = 0.58778525229247312917;
+    const float2 a1 = cadd(x[1], x[4]), b1 = csub(x[1], x[4]);
+    const float2 a2 = cadd(x[2], x[3]), b2 = csub(x[2], x[3]);
+    const float2 x0 = x[0];
+    const float2 m1 = cadd(x0, lin2<true>(c1, a1, c2, a2)), m2 = cadd(x0, lin2<true>(c2, a1, c1, a2));
+    const float2 n1 = rot<DIR>(lin2<true>(s1, b1, s2, b2)), n2 = rot<DIR>(lin2<true>(s2, b1, -s1, b2));
+    x[0] = cadd(x0, cadd(a1, a2));
+    x[1] = cadd(m1, n1);
+    x[4] = csub(m1, n1);
+    x[2] = cadd(m2, n2);
+    x[3] = csub(m2, n2);
+    return;
+  }
   constexpr float c1 = 0.30901699437494742410f;   // cos(2 pi/5)
   constexpr float c2 = -0.80901699437494742410f;  // cos(4 pi/5)
   constexpr float s1 = 0.95105651629515357212f;   // sin(2 pi/5)
@@ -372,50 +434,53 @@ __device__ __forceinline__ void dft7(float2* x) {
   x[4] = csub(m3, n3);
 }
 
-template <int R, int DIR>
+template <int R, int DIR, bool COMP = false>
 __device__ __forceinline__ void dft(float2* x);
 
 // (cos, sin) of 2 pi m / R, 0 < m < R, for the composite radices
+struct Root {
+  double c, s;
+};
 template <int R>
-__device__ __forceinline__ float2 unit_root(int m) {
+__device__ __forceinline__ Root unit_root(int m) {
   if constexpr (R == 6) {
-    constexpr float c[6] = {1.f, 0.5f, -0.5f, -1.f, -0.5f, 0.5f};
-    constexpr float s[6] = {0.f, 0.86602540378443864676f, 0.86602540378443864676f, 0.f, -0.86602540378443864676f,
-                            -0.86602540378443864676f};
-    return make_float2(c[m], s[m]);
+    constexpr double c[6] = {1., 0.5, -0.5, -1., -0.5, 0.5};
+    constexpr double s[6] = {0., 0.86602540378443864676, 0.86602540378443864676, 0., -0.86602540378443864676,
+                            -0.86602540378443864676};
+    return Root{c[m], s[m]};
   } else if constexpr (R == 9) {
-    constexpr float c[9] = {1.f, 0.76604444311897803520f, 0.17364817766693034885f, -0.5f, -0.93969262078590838405f,
-                            -0.93969262078590838405f, -0.5f, 0.17364817766693034885f, 0.76604444311897803520f};
-    constexpr float s[9] = {0.f, 0.64278760968653932632f, 0.98480775301220805936f, 0.86602540378443864676f,
-                            0.34202014332566873304f, -0.34202014332566873304f, -0.86602540378443864676f,
-                            -0.98480775301220805936f, -0.64278760968653932632f};
-    return make_float2(c[m], s[m]);
+    constexpr double c[9] = {1., 0.76604444311897803520, 0.17364817766693034885, -0.5, -0.93969262078590838405,
+                            -0.93969262078590838405, -0.5, 0.17364817766693034885, 0.76604444311897803520};
+    constexpr double s[9] = {0., 0.64278760968653932632, 0.98480775301220805936, 0.86602540378443864676,
+                            0.34202014332566873304, -0.34202014332566873304, -0.86602540378443864676,
+                            -0.98480775301220805936, -0.64278760968653932632};
+    return Root{c[m], s[m]};
   } else if constexpr (R == 10) {
-    constexpr float c[10] = {1.f, 0.80901699437494742410f, 0.30901699437494742410f, -0.30901699437494742410f,
-                             -0.80901699437494742410f, -1.f, -0.80901699437494742410f, -0.30901699437494742410f,
-                             0.30901699437494742410f, 0.80901699437494742410f};
-    constexpr float s[10] = {0.f, 0.58778525229247312917f, 0.95105651629515357212f, 0.95105651629515357212f,
-                             0.58778525229247312917f, 0.f, -0.58778525229247312917f, -0.95105651629515357212f,
-                             -0.95105651629515357212f, -0.58778525229247312917f};
-    return make_float2(c[m], s[m]);
+    constexpr double c[10] = {1., 0.80901699437494742410, 0.30901699437494742410, -0.30901699437494742410,
+                             -0.80901699437494742410, -1., -0.80901699437494742410, -0.30901699437494742410,
+                             0.30901699437494742410, 0.80901699437494742410};
+    constexpr double s[10] = {0., 0.58778525229247312917, 0.95105651629515357212, 0.95105651629515357212,
+                             0.58778525229247312917, 0., -0.58778525229247312917, -0.95105651629515357212,
+                             -0.95105651629515357212, -0.58778525229247312917};
+    return Root{c[m], s[m]};
   } else if constexpr (R == 12) {
-    constexpr float c[12] = {1.f, 0.86602540378443864676f, 0.5f, 0.f, -0.5f, -0.86602540378443864676f, -1.f,
-                             -0.86602540378443864676f, -0.5f, 0.f, 0.5f, 0.86602540378443864676f};
-    constexpr float s[12] = {0.f, 0.5f, 0.86602540378443864676f, 1.f, 0.86602540378443864676f, 0.5f, 0.f, -0.5f,
-                             -0.86602540378443864676f, -1.f, -0.86602540378443864676f, -0.5f};
-    return make_float2(c[m], s[m]);
+    constexpr double c[12] = {1., 0.86602540378443864676, 0.5, 0., -0.5, -0.86602540378443864676, -1.,
+                             -0.86602540378443864676, -0.5, 0., 0.5, 0.86602540378443864676};
+    constexpr double s[12] = {0., 0.5, 0.86602540378443864676, 1., 0.86602540378443864676, 0.5, 0., -0.5,
+                             -0.86602540378443864676, -1., -0.86602540378443864676, -0.5};
+    return Root{c[m], s[m]};
   } else {
     static_assert(R == 15, "no table for this radix");
-    constexpr float c[15] = {1.f, 0.91354545764260089550f, 0.66913060635885821383f, 0.30901699437494742410f,
-                             -0.10452846326765347140f, -0.5f, -0.80901699437494742410f, -0.97814760073380563793f,
-                             -0.97814760073380563793f, -0.80901699437494742410f, -0.5f, -0.10452846326765347140f,
-                             0.30901699437494742410f, 0.66913060635885821383f, 0.91354545764260089550f};
-    constexpr float s[15] = {0.f, 0.40673664307580020775f, 0.74314482547739423501f, 0.95105651629515357212f,
-                             0.99452189536827333692f, 0.86602540378443864676f, 0.58778525229247312917f,
-                             0.20791169081775933710f, -0.20791169081775933710f, -0.58778525229247312917f,
-                             -0.86602540378443864676f, -0.99452189536827333692f, -0.95105651629515357212f,
-                             -0.74314482547739423501f, -0.40673664307580020775f};
-    return make_float2(c[m], s[m]);
+    constexpr double c[15] = {1., 0.91354545764260089550, 0.66913060635885821383, 0.30901699437494742410,
+                             -0.10452846326765347140, -0.5, -0.80901699437494742410, -0.97814760073380563793,
+                             -0.97814760073380563793, -0.80901699437494742410, -0.5, -0.10452846326765347140,
+                             0.30901699437494742410, 0.66913060635885821383, 0.91354545764260089550};
+    constexpr double s[15] = {0., 0.40673664307580020775, 0.74314482547739423501, 0.95105651629515357212,
+                             0.99452189536827333692, 0.86602540378443864676, 0.58778525229247312917,
+                             0.20791169081775933710, -0.20791169081775933710, -0.58778525229247312917,
+                             -0.86602540378443864676, -0.99452189536827333692, -0.95105651629515357212,
+                             -0.74314482547739423501, -0.40673664307580020775};
+    return Root{c[m], s[m]};
   }
 }
 
@@ -423,7 +488,7 @@ __device__ __forceinline__ float2 unit_root(int m) {
 // DFTs of the R1 subsequences x[n1 + R1 n2], the twiddles
 // exp(DIR 2 pi i n1 k2 / R), then R1-point DFTs; X[R2 k1 + k2] comes out in
 // natural order.
-template <int R1, int R2, int DIR>
+template <int R1, int R2, int DIR, bool COMP = false>
 __device__ __forceinline__ void dft_ct(float2* x) {
   constexpr int R = R1 * R2;
   float2 y[R];
@@ -432,15 +497,15 @@ __device__ __forceinline__ void dft_ct(float2* x) {
     float2 c[R2];
 #pragma unroll
     for (int n2 = 0; n2 < R2; ++n2) c[n2] = x[n1 + R1 * n2];
-    dft<R2, DIR>(c);
+    dft<R2, DIR, COMP>(c);
 #pragma unroll
     for (int k2 = 0; k2 < R2; ++k2) {
       const int m = n1 * k2;
       if (m == 0) {
         y[n1 * R2 + k2] = c[k2];
       } else {
-        const float2 w = unit_root<R>(m);
-        y[n1 * R2 + k2] = make_float2(c[k2].x * w.x - DIR * c[k2].y * w.y, c[k2].y * w.x + DIR * c[k2].x * w.y);
+        const Root w = unit_root<R>(m);
+        y[n1 * R2 + k2] = rotc<DIR, COMP>(c[k2], w.c, w.s);
       }
     }
   }
@@ -449,26 +514,26 @@ __device__ __forceinline__ void dft_ct(float2* x) {
     float2 r[R1];
 #pragma unroll
     for (int n1 = 0; n1 < R1; ++n1) r[n1] = y[n1 * R2 + k2];
-    dft<R1, DIR>(r);
+    dft<R1, DIR, COMP>(r);
 #pragma unroll
     for (int k1 = 0; k1 < R1; ++k1) x[R2 * k1 + k2] = r[k1];
   }
 }
 
-template <int R, int DIR>
+template <int R, int DIR, bool COMP>
 __device__ __forceinline__ void dft(float2* x) {
   if constexpr (R == 2) dft2<DIR>(x[0], x[1]);
-  else if constexpr (R == 3) dft3<DIR>(x);
+  else if constexpr (R == 3) dft3<DIR, COMP>(x);
   else if constexpr (R == 4) dft4<DIR>(x[0], x[1], x[2], x[3]);
-  else if constexpr (R == 5) dft5<DIR>(x);
-  else if constexpr (R == 6) dft_ct<2, 3, DIR>(x);
+  else if constexpr (R == 5) dft5<DIR, COMP>(x);
+  else if constexpr (R == 6) dft_ct<2, 3, DIR, COMP>(x);
   else if constexpr (R == 7) dft7<DIR>(x);
-  else if constexpr (R == 8) dft8<DIR>(x);
-  else if constexpr (R == 9) dft_ct<3, 3, DIR>(x);
-  else if constexpr (R == 10) dft_ct<2, 5, DIR>(x);
-  else if constexpr (R == 12) dft_ct<4, 3, DIR>(x);
-  else if constexpr (R == 15) dft_ct<3, 5, DIR>(x);
-  else if constexpr (R == 16) dft16<DIR>(x);
+  else if constexpr (R == 8) dft8<DIR, COMP>(x);
+  else if constexpr (R == 9) dft_ct<3, 3, DIR, COMP>(x);
+  else if constexpr (R == 10) dft_ct<2, 5, DIR, COMP>(x);
+  else if constexpr (R == 12) dft_ct<4, 3, DIR, COMP>(x);
+  else if constexpr (R == 15) dft_ct<3, 5, DIR, COMP>(x);
+  else if constexpr (R == 16) dft16<DIR, COMP>(x);
   else static_assert(R == 2, "unsupported radix");
 }
 
