@@ -73,6 +73,9 @@ struct Shape {
   const float2 *volr_tw = nullptr, *volc_tw = nullptr;
 };
 int make_shape(int nx, int ny, int nz, int nrec, Shape* sh);
+// a one-reconstruction shape's transforms over nrec reconstructions (its
+// iterations keep the layout choices of one)
+Shape shape_of_many(const Shape& one, int nrec);
 // elements per thread (4, 8 or 16; 0 for a trivial axis) of the x, y and z
 // transform variants chosen for arrays of shape (nz, ny, nx), tuning the
 // shape on its first use

@@ -1372,6 +1372,14 @@ int make_shape(int nx, int ny, int nz, int nrec, Shape* sh) {
   return 0;
 }
 
+Shape shape_of_many(const Shape& one, int nrec) {
+  Shape sh = one;
+  sh.nrec = nrec;
+  sh.gy.nouter = one.nz * nrec;
+  for (LineGeom* g : {&sh.gz, &sh.gyt, &sh.gytr}) g->nouter = nrec;
+  return sh;
+}
+
 int shape_variant_elements(int nx, int ny, int nz, int* e) {
   Shape sh;
   if (int rc = make_shape(nx, ny, nz, 1, &sh)) return rc;
@@ -1492,10 +1500,7 @@ static int tune_volume_hints(const Shape& sh0) {
   int nr = batch_class(sh0.nrec) == 3 && sh0.nrec < 16 ? 16 : sh0.nrec;
   if ((long)nr * N > (1L << 24)) nr = (int)((1L << 24) / N);
   if (nr < 1) nr = 1;
-  Shape sh = sh0;
-  sh.nrec = nr;
-  sh.gy = LineGeom{sh.nx, sh.nz * nr, (long)sh.nx * sh.ny, (long)sh.nx};
-  sh.gz = LineGeom{sh.nx * sh.ny, nr, N, (long)sh.nx * sh.ny};
+  const Shape sh = shape_of_many(sh0, nr);
   const long n = (long)nr * N;
   hipStream_t s = nullptr;
   float2 *w = nullptr, *g0 = nullptr, *g1 = nullptr;
