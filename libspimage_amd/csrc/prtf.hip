@@ -400,14 +400,16 @@ int prtf_impl(const float* images, const int* masks, int nx, int ny, int nz, int
   float* dprtf = reinterpret_cast<float*>(t1);
   hipLaunchKernelGGL(k_prtf_final, g, blk, 0, s, sum, zeros, dprtf, N, (float)n);
   SPX_HIP(hipGetLastError());
-  SPX_HIP(hipMemcpyAsync(prtf, dprtf, sizeof(float) * N, hipMemcpyDeviceToHost, s));
-  if (super_image) SPX_HIP(hipMemcpyAsync(super_image, avg, sizeof(float2) * N, hipMemcpyDeviceToHost, s));
+  if (int rc = download_d2h(prtf, dprtf, sizeof(float) * N, s)) return rc;
+  if (super_image)
+    if (int rc = download_d2h(super_image, avg, sizeof(float2) * N, s)) return rc;
   if (aligned) SPX_HIP(hipMemcpyAsync(aligned, imgs, sizeof(float2) * n * N, hipMemcpyDeviceToHost, s));
   if (aligned_masks) {
     if (msk) SPX_HIP(hipMemcpyAsync(aligned_masks, amsk ? amsk : msk, sizeof(int) * n * N, hipMemcpyDeviceToHost, s));
     else memset(aligned_masks, 0, sizeof(int) * n * N);
   }
-  if (mask_count) SPX_HIP(hipMemcpyAsync(mask_count, cnt, sizeof(float) * N, hipMemcpyDeviceToHost, s));
+  if (mask_count)
+    if (int rc = download_d2h(mask_count, cnt, sizeof(float) * N, s)) return rc;
   SPX_HIP(hipStreamSynchronize(s));
   return 0;
 }
