@@ -71,11 +71,12 @@ __global__ __launch_bounds__((ColShape<M, E>::NT)) void k_any_col(ColArgs a, Any
     __syncthreads();
     any_line<M, E>(v, true, va, vb, t, tw, ch);
   } else if constexpr (MODE == kColBlur) {
+    const BlurLine blur(a, base);
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
       if (!low_reg<M, E>(q)) continue;
       const int p = in_pos<M, E>(t, q);
-      const float h = p < c.L ? blur_transfer(a, base + p * st) : 0.f;
+      const float h = p < c.L ? blur.at(p) : 0.f;
       v[q] = p < c.L ? make_float2(v[q].x * h, v[q].y * h) : make_float2(0.f, 0.f);
     }
     __syncthreads();

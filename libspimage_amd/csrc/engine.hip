@@ -824,8 +824,15 @@ __global__ __launch_bounds__(kRedThreads) void k_sumsq_f32(const float* in, long
 }
 
 __global__ __launch_bounds__(kRedThreads) void k_count_support(const uint8_t* flags, long n, double* partials) {
-  double acc[1] = {0.0};
-  REC_STRIDE(i, n) acc[0] += (flags[i] & kInsideSupport) ? 1.0 : 0.0;
+  unsigned c = 0;  // a thread's share of fewer than 2^31 pixels
+  if ((n & 15) == 0) {
+    constexpr unsigned m = kInsideSupport * 0x01010101u;
+    const uint4* f = reinterpret_cast<const uint4*>(flags);
+    REC_STRIDE(i, n >> 4) c += __popc(f[i].x & m) + __popc(f[i].y & m) + __popc(f[i].z & m) + __popc(f[i].w & m);
+  } else {
+    REC_STRIDE(i, n) c += (flags[i] & kInsideSupport) ? 1u : 0u;
+  }
+  double acc[1] = {(double)c};
   write_partials<1>(acc, partials);
 }
 
@@ -851,99 +858,162 @@ __global__ __launch_bounds__(256) void k_reduce_rec(const double* partials, int 
 // --- reference's qsort-then-index, src/support_update.c:143-144) by a
 // --- three-level radix select over the float bit patterns (non-negative
 // --- floats order like their bits): 11 + 11 + 10 bits.
-__global__ void k_ctl_init(unsigned* ctl, int nrec, unsigned k) {
-  for (int r = threadIdx.x; r < nrec; r += blockDim.x) {
-    unsigned* c = ctl + r * kCtlStride;
-    c[kCtlK] = k;
-    c[kCtlPrefix] = 0;
-    c[kCtlThresh] = 0;
-    for (int x = 0; x < kHistSlices; ++x) c[kCtlMax + x] = 0;
-  }
+// These kernels are bound by their launches (6-7 us each with the gap) and
+// by the latency of few loads a thread, so the bins of levels 2 and 3 are
+// picked at the start of the kernel that needs them, by every block for itself
+// (8 and 4 KB from L2), and arrays are read four pixels at a time.  Level 1
+// (64 KB in its copies) keeps its own launch.  1024^2 from the histogram's
+// clearing to the mask: 38 us of kernels in 8
+// launches -> 20 us in 5.
+__global__ void k_ctl_init(unsigned* ctl, int nrec) {
+  for (int r = threadIdx.x; r < nrec; r += blockDim.x)
+    for (int x = 0; x < kHistSlices; ++x) ctl[r * kCtlStride + kCtlMax + x] = 0;
 }
 
-// one block per reconstruction
-__global__ __launch_bounds__(1024) void k_select(const unsigned* hist_all, int level, unsigned* ctl_all) {
-  __shared__ unsigned scan[1024];
-  __shared__ unsigned lvl1[2048];
-  const int nbins = (level == 3) ? 1024 : 2048;
-  const unsigned* hist =
-      hist_all + (long)blockIdx.x * kHistStride + (level == 1 ? 0 : level == 2 ? kHistLevel2 : kHistLevel3);
-  unsigned* ctl = ctl_all + blockIdx.x * kCtlStride;
-  const int per = nbins / 1024;  // 1 or 2 bins per thread, walked high to low
-  const int tid = threadIdx.x;
-  if (level == 1) {
-    // the per-XCD copies of the level-1 histogram, summed
-    for (int b = tid; b < 2048; b += 1024) {
-      unsigned c = 0;
-      for (int x = 0; x < kHistSlices; ++x) c += hist[x * 2048 + b];
-      lvl1[b] = c;
+constexpr int kSelThreads = 256;
+struct Pick {
+  unsigned bin, k;  // the bin that holds descending index k of the histogram, the index within it
+};
+// All threads of the block return the same; `slices` copies of 2048 bins are
+// summed.  Scans by wavefront, high bins first.
+template <int NBINS, int SLICES>
+__device__ __forceinline__ Pick pick_bin(const unsigned* hist, unsigned k) {
+  constexpr int PER = NBINS / kSelThreads, NW = kSelThreads / 64;
+  static_assert(PER % 4 == 0, "whole vectors of bins");
+  __shared__ unsigned waves[NW];
+  __shared__ Pick found;
+  const int tid = threadIdx.x, lo = NBINS - (tid + 1) * PER;
+  unsigned c[PER] = {};
+#pragma unroll
+  for (int x = 0; x < SLICES; ++x)
+#pragma unroll
+    for (int q = 0; q < PER; q += 4) {
+      const uint4 v = *reinterpret_cast<const uint4*>(&hist[x * 2048 + lo + q]);
+      c[q] += v.x;
+      c[q + 1] += v.y;
+      c[q + 2] += v.z;
+      c[q + 3] += v.w;
     }
-    __syncthreads();
-    hist = lvl1;
-  }
-  const unsigned k = ctl[kCtlK];
   unsigned local = 0;
-  for (int q = 0; q < per; ++q) local += hist[nbins - 1 - (tid * per + q)];
-  scan[tid] = local;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const unsigned v = (tid >= off) ? scan[tid - off] : 0u;
-    __syncthreads();
-    scan[tid] += v;
-    __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PER; ++q) local += c[q];
+  unsigned before = local;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const unsigned v = __shfl_up(before, off, 64);
+    if ((tid & 63) >= off) before += v;
   }
-  unsigned before = scan[tid] - local;  // elements in strictly higher bins
-  const unsigned prefix = ctl[kCtlPrefix];
+  if ((tid & 63) == 63) waves[tid >> 6] = before;
+  before -= local;
+  if (tid == 0) found = Pick{0, 0};
   __syncthreads();
-  for (int q = 0; q < per; ++q) {
-    const int b = nbins - 1 - (tid * per + q);
-    const unsigned c = hist[b];
-    if (c > 0 && before <= k && k < before + c) {
-      ctl[kCtlK] = k - before;
-      if (level == 1) ctl[kCtlPrefix] = (unsigned)b;
-      else if (level == 2) ctl[kCtlPrefix] = (prefix << 11) | (unsigned)b;
-      else ctl[kCtlThresh] = (prefix << 10) | (unsigned)b;
-    }
-    before += c;
+#pragma unroll
+  for (int w = 0; w < NW - 1; ++w) before += (tid >> 6) > w ? waves[w] : 0u;
+#pragma unroll
+  for (int q = PER - 1; q >= 0; --q) {
+    if (c[q] > 0 && before <= k && k < before + c[q]) found = Pick{(unsigned)(lo + q), k - before};
+    before += c[q];
+  }
+  __syncthreads();
+  return found;
+}
+
+// f(pixel index, |blur|) over a reconstruction's pixels, four at a time where
+// they are whole 16-byte vectors
+template <class F4, class F>
+__device__ __forceinline__ void each_abs(const float* absb, long n, F4&& f4, F&& f) {
+  if ((n & 3) == 0) {
+    const float4* v = reinterpret_cast<const float4*>(absb);
+    REC_STRIDE(i, n >> 2) f4(i, v[i]);
+  } else {
+    REC_STRIDE(i, n) f(i, absb[i]);
   }
 }
 
-// grid (blocks_per_rec, nrec)
-__global__ __launch_bounds__(256) void k_hist_level(const float* absb, long n, unsigned* hist_all, const unsigned* ctl_all,
-                                                    int level) {
-  __shared__ unsigned h[2048];
-  const int nb = (level == 2) ? 2048 : 1024;
-  unsigned* hist = hist_all + (long)blockIdx.y * kHistStride + (level == 2 ? kHistLevel2 : kHistLevel3);
-  for (int i = threadIdx.x; i < nb; i += blockDim.x) h[i] = 0u;
+// level 1: one block per reconstruction
+__global__ __launch_bounds__(kSelThreads) void k_select(const unsigned* hist_all, unsigned* ctl_all, unsigned k) {
+  unsigned* ctl = ctl_all + blockIdx.x * kCtlStride;
+  const Pick p = pick_bin<2048, kHistSlices>(hist_all + (long)blockIdx.x * kHistStride, k);
+  if (threadIdx.x == 0) {
+    ctl[kCtlK] = p.k;
+    ctl[kCtlPrefix] = p.bin;
+  }
+}
+
+// Counts of level 2 (bits 20..10 of the values in level 1's bin) or 3 (bits
+// 9..0 of those in level 2's).  Grid (blocks_per_rec, nrec).
+template <int LEVEL>
+__global__ __launch_bounds__(kSelThreads) void k_hist_level(const float* absb, long n, unsigned* hist_all,
+                                                            unsigned* ctl_all) {
+  constexpr int NB = LEVEL == 2 ? 2048 : 1024;
+  __shared__ unsigned h[NB];
+  unsigned* hist = hist_all + (long)blockIdx.y * kHistStride;
+  unsigned* ctl = ctl_all + blockIdx.y * kCtlStride;
+  for (int i = threadIdx.x; i < NB; i += kSelThreads) h[i] = 0u;
+  unsigned pre = ctl[kCtlPrefix];
+  if constexpr (LEVEL == 3) {
+    const Pick p = pick_bin<2048, 1>(hist + kHistLevel2, ctl[kCtlK]);
+    pre = (pre << 11) | p.bin;
+    // other slots than those that the other blocks still read
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      ctl[kCtlK2] = p.k;
+      ctl[kCtlPrefix2] = pre;
+    }
+    hist += kHistLevel3;
+  } else {
+    hist += kHistLevel2;
+  }
   __syncthreads();
-  const unsigned pre = ctl_all[blockIdx.y * kCtlStride + kCtlPrefix];
-  REC_STRIDE(i, n) {
-    const unsigned b = __float_as_uint(absb[i]);
-    if (level == 2) {
+  const auto count = [&](float m) {
+    const unsigned b = __float_as_uint(m);
+    if constexpr (LEVEL == 2) {
       if ((b >> 21) == pre) atomicAdd(&h[(b >> 10) & 2047u], 1u);
     } else {
       if ((b >> 10) == pre) atomicAdd(&h[b & 1023u], 1u);
     }
-  }
+  };
+  each_abs(
+      absb, n,
+      [&](long, float4 m) {
+        count(m.x);
+        count(m.y);
+        count(m.z);
+        count(m.w);
+      },
+      [&](long, float m) { count(m); });
   __syncthreads();
-  for (int i = threadIdx.x; i < nb; i += blockDim.x)
+  for (int i = threadIdx.x; i < NB; i += kSelThreads)
     if (h[i]) atomicAdd(&hist[i], h[i]);
 }
 
-// support bit = |blur| > threshold (reference src/support_update.c:392-400);
-// mode 0: threshold = selected value, mode 1: max * rel
-// (src/support_update.c:175).  Grid (blocks_per_rec, nrec).
-__global__ void k_mask(const float* absb, uint8_t* flags, long n, unsigned* ctl_all, int mode, float rel) {
+// support bit = |blur| > threshold (reference src/support_update.c:392-400):
+// the value the select ends at, picked from its level-3 histogram, or (hist
+// null) the running maximum * rel (src/support_update.c:175).  Grid
+// (blocks_per_rec, nrec).
+__global__ __launch_bounds__(kSelThreads) void k_mask(const float* absb, uint8_t* flags, long n, const unsigned* hist_all,
+                                                      unsigned* ctl_all, float rel) {
   unsigned* ctl = ctl_all + blockIdx.y * kCtlStride;
-  unsigned mx = 0;
-  for (int x = 0; x < kHistSlices; ++x) mx = (ctl[kCtlMax + x] > mx) ? ctl[kCtlMax + x] : mx;
-  const float t = (mode == 0) ? __uint_as_float(ctl[kCtlThresh]) : __uint_as_float(mx) * rel;
-  // record the threshold of mode 1 (mode 0 already holds it in kCtlThresh)
-  if (mode == 1 && blockIdx.x == 0 && threadIdx.x == 0) ctl[kCtlThresh] = __float_as_uint(t);
-  REC_STRIDE(i, n) {
-    const uint8_t f = flags[i];
-    flags[i] = (absb[i] > t) ? (uint8_t)(f | kInsideSupport) : (uint8_t)(f & ~kInsideSupport);
+  float t;
+  if (hist_all) {
+    const Pick p = pick_bin<1024, 1>(hist_all + (long)blockIdx.y * kHistStride + kHistLevel3, ctl[kCtlK2]);
+    t = __uint_as_float((ctl[kCtlPrefix2] << 10) | p.bin);
+  } else {
+    unsigned mx = 0;
+    for (int x = 0; x < kHistSlices; ++x) mx = (ctl[kCtlMax + x] > mx) ? ctl[kCtlMax + x] : mx;
+    t = __uint_as_float(mx) * rel;
   }
+  if (blockIdx.x == 0 && threadIdx.x == 0) ctl[kCtlThresh] = __float_as_uint(t);
+  const auto bit = [t](uint8_t f, float m) {
+    return (m > t) ? (uint8_t)(f | kInsideSupport) : (uint8_t)(f & ~kInsideSupport);
+  };
+  uchar4* flags4 = reinterpret_cast<uchar4*>(flags);
+  each_abs(
+      absb, n,
+      [&](long i, float4 m) {
+        const uchar4 f = flags4[i];
+        flags4[i] = make_uchar4(bit(f.x, m.x), bit(f.y, m.y), bit(f.z, m.z), bit(f.w, m.w));
+      },
+      [&](long i, float m) { flags[i] = bit(flags[i], m); });
 }
 
 // One pass of the support closing (reference src/support_update.c:213-280):
@@ -2523,14 +2593,12 @@ int Engine::shrinkwrap_area(float sigma, float area) {
   const int bpr = rec_blocks(N);
   const long nh = (long)kHistStride * nrec;
   hipLaunchKernelGGL(k_fill_u32, ew_grid(nh), dim3(256), 0, s, hist, nh, 0u);
-  hipLaunchKernelGGL(k_ctl_init, dim3(1), dim3(256), 0, s, ctl, nrec, (unsigned)k);
   if (int rc = blur_to_abs(sigma, true)) return rc;
-  hipLaunchKernelGGL(k_select, dim3(nrec), dim3(1024), 0, s, hist, 1, ctl);
-  hipLaunchKernelGGL(k_hist_level, dim3(bpr, nrec), dim3(256), 0, s, absb, N, hist, ctl, 2);
-  hipLaunchKernelGGL(k_select, dim3(nrec), dim3(1024), 0, s, hist, 2, ctl);
-  hipLaunchKernelGGL(k_hist_level, dim3(bpr, nrec), dim3(256), 0, s, absb, N, hist, ctl, 3);
-  hipLaunchKernelGGL(k_select, dim3(nrec), dim3(1024), 0, s, hist, 3, ctl);
-  hipLaunchKernelGGL(k_mask, dim3(bpr, nrec), dim3(256), 0, s, absb, flags, N, ctl, 0, 0.f);
+  const dim3 grid(bpr, nrec), blk(kSelThreads);
+  hipLaunchKernelGGL(k_select, dim3(nrec), blk, 0, s, hist, ctl, (unsigned)k);
+  hipLaunchKernelGGL(k_hist_level<2>, grid, blk, 0, s, absb, N, hist, ctl);
+  hipLaunchKernelGGL(k_hist_level<3>, grid, blk, 0, s, absb, N, hist, ctl);
+  hipLaunchKernelGGL(k_mask, grid, blk, 0, s, absb, flags, N, hist, ctl, 0.f);
   SPX_HIP(hipGetLastError());
   ++flags_version;
   return 0;
@@ -2544,9 +2612,9 @@ int Engine::last_threshold(float* t) {
 }
 
 int Engine::shrinkwrap_threshold(float sigma, float rel) {
-  hipLaunchKernelGGL(k_ctl_init, dim3(1), dim3(256), 0, s, ctl, nrec, 0u);
+  hipLaunchKernelGGL(k_ctl_init, dim3(1), dim3(256), 0, s, ctl, nrec);
   if (int rc = blur_to_abs(sigma, false)) return rc;
-  hipLaunchKernelGGL(k_mask, dim3(rec_blocks(N), nrec), dim3(256), 0, s, absb, flags, N, ctl, 1, rel);
+  hipLaunchKernelGGL(k_mask, dim3(rec_blocks(N), nrec), dim3(kSelThreads), 0, s, absb, flags, N, (const unsigned*)nullptr, ctl, rel);
   SPX_HIP(hipGetLastError());
   ++flags_version;
   return 0;
@@ -2618,12 +2686,12 @@ int Engine::patterson_support(const float* amp_raw, float value) {
     c.geo = sh.gz;
     sh.ez->col(kColInv, c, s);
   }
-  hipLaunchKernelGGL(k_ctl_init, dim3(1), dim3(256), 0, s, ctl, nrec, 0u);
+  hipLaunchKernelGGL(k_ctl_init, dim3(1), dim3(256), 0, s, ctl, nrec);
   RowArgs r = row_args(sh, S1, nullptr);
   r.absb = absb;
   r.ctl = ctl;
   sh.ex->row(kRowBlurOut, r, s);
-  hipLaunchKernelGGL(k_mask, dim3(rec_blocks(N), nrec), dim3(256), 0, s, absb, flags, N, ctl, 1, value);
+  hipLaunchKernelGGL(k_mask, dim3(rec_blocks(N), nrec), dim3(kSelThreads), 0, s, absb, flags, N, (const unsigned*)nullptr, ctl, value);
   SPX_HIP(hipGetLastError());
   SPX_HIP(hipStreamSynchronize(s));
   ++flags_version;

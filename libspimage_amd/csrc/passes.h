@@ -122,7 +122,8 @@ constexpr int kCtlStride = 16;
 // (x | y << 16 in slot 6, z in slot 7), each wrapped into [0, n).
 enum CtlSlot {
   kCtlK = 0, kCtlPrefix = 1, kCtlThresh = 2, kCtlCentre = 3 /* .. 5 */, kCtlCentreShift = 6 /* .. 7 */,
-  kCtlMax = 8 /* .. 15, one per XCD */
+  kCtlMax = 8 /* .. 15, one per XCD */,
+  kCtlK2 = 8, kCtlPrefix2 = 9  // the area update, which keeps no maxima: k and prefix after level 2
 };
 
 struct RowArgs {
@@ -279,24 +280,36 @@ struct SupportConstraints {
 };
 
 // Gaussian transfer function of sp_gaussian_blur (src/image_filter.c:80-91)
-// with dist_to_top_left (src/image_util.c:1012-1032) at index idx of the
-// reconstruction-stacked array, computed in double and rounded to float like
-// the reference.
-__device__ __forceinline__ float blur_transfer(const ColArgs& a, long idx) {
-  const double NN = (double)((float)((long)a.nx * a.ny * a.nz));
-  const double k0 = -2.0 * (3.14159265358979323846 * 3.14159265358979323846);
-  const double s2 = (double)a.sigma * (double)a.sigma;
-  const int ix = (int)(idx % a.nx);
-  const long rest = idx / a.nx;
-  const int iy = (int)(rest % a.ny);
-  const int iz = (int)((rest / a.ny) % a.nz);  // reconstructions stack along z
-  const float dx = (a.nx - ix < ix) ? (float)(a.nx - ix) : (float)ix;
-  const float dy = (a.ny - iy < iy) ? (float)(a.ny - iy) : (float)iy;
-  const float dz = (a.nz - iz < iz) ? (float)(a.nz - iz) : (float)iz;
-  const float dist = (float)sqrt((double)dx * dx + (double)dy * dy + (double)dz * dz);
-  const float r = dist / (float)a.nx;
-  return (float)(exp(k0 * ((double)r * (double)r) * s2) / NN);
-}
+// with dist_to_top_left (src/image_util.c:1012-1032) along one line of the
+// row-major reconstruction-stacked array whose first element is `base`,
+// computed in double and rounded to float like the reference.  The line's
+// coordinates are taken from `base` once: their 64-bit divisions for every
+// pixel were most of the pass (1024^2: 23.1 us with them, 15.1 us without,
+// same bits).
+struct BlurLine {
+  double across, NN, s2;  // squared distance across the line
+  int n;                  // its length
+  float nx;
+  __device__ __forceinline__ BlurLine(const ColArgs& a, long base) {
+    const int ix = (int)(base % a.nx);
+    const long rest = base / a.nx;
+    const bool along_y = a.ny > 1 && a.geo.axis_stride == a.nx;
+    // reconstructions stack along z
+    const int io = along_y ? (int)((rest / a.ny) % a.nz) : (int)(rest % a.ny), no = along_y ? a.nz : a.ny;
+    const double dx = (a.nx - ix < ix) ? a.nx - ix : ix, dn = (no - io < io) ? no - io : io;
+    across = dx * dx + dn * dn;
+    NN = (double)((float)((long)a.nx * a.ny * a.nz));
+    s2 = (double)a.sigma * (double)a.sigma;
+    n = along_y ? a.ny : a.nz;
+    nx = (float)a.nx;
+  }
+  __device__ __forceinline__ float at(int i) const {
+    const double k0 = -2.0 * (3.14159265358979323846 * 3.14159265358979323846);
+    const double d = (n - i < i) ? n - i : i;
+    const float r = (float)sqrt(across + d * d) / nx;
+    return (float)(exp(k0 * ((double)r * (double)r) * s2) / NN);
+  }
+};
 
 // One pixel's terms of the E_F sums (src/phasing.c:879-888): measured pixels
 // add (|F|-|amp|)^2 and amp^2, unmeasured ones |F|^2; FcFo sums |amp| and |F|
@@ -921,10 +934,11 @@ __global__ __launch_bounds__((ColShape<L, E, WIDE>::NT)) void k_col(ColArgs a) {
     __syncthreads();
     fft_line<L, E, +1>(v, va, vb, t, twr);
   } else if constexpr (MODE == kColBlur) {
+    const BlurLine blur(a, base);
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
       if (!act) continue;
-      const float h = blur_transfer(a, base + out_pos<L, E>(t, q) * st);
+      const float h = blur.at(out_pos<L, E>(t, q));
       v[q] = make_float2(v[q].x * h, v[q].y * h);
     }
     out_to_in<L, E>(v, va, t);
