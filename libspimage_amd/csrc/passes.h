@@ -477,26 +477,42 @@ __global__ __launch_bounds__((RowShape<L, E>::NT)) void k_row(RowArgs a) {
 // update runs on registers at the inverse transform's output positions; its
 // other operands (g_k, flags) are loaded before the inverse transform.
 // Thread layout of row work-groups.  Natural layout: M lines of T threads
-// each (thread = line * T + t).  4-column tiled layout of W: 4 consecutive
-// lines whose lanes interleave as 16 positions x 4 lines, so that one
-// wavefront load covers 16 consecutive x of 4 rows: four whole 128-byte
-// lines of a row-major array and four whole 4 x 4 tiles of the tiled one.
+// each (thread = line * T + t).  4-column tiled layout of W: 4 or 2
+// consecutive lines whose lanes interleave as 16 positions x M lines, so that
+// one wavefront load covers whole 128-byte lines of a row-major array and
+// whole 4 x 4 tiles (or halves, which the neighbouring work-group on the same
+// XCD completes in its L2) of the tiled one.
+//
+// 2 lines where 4 leave one work-group a CU (kOneGroup: 1215 points and more but for 2352 to 2401):
+// nothing else then loads or stores while it transforms.  Microseconds per HIO
+// iteration with 4 and with 2 lines (and the column pass's pairs, ColShape):
+// 2048^2 60.9 -> 51.4, in batches of 4 199 -> 169; 3072^2 151 -> 138; 4096^2
+// 260 (transposed) -> 237.  Shorter lines keep 4: 1024^2 with E = 8 and 2
+// lines ran 17.5 -> 16.7 us in the tuner but 14.3 -> 15.1 in a phaser.
+template <int L>
+struct LineLds {
+  static constexpr int LS = L + (L >> 4);
+  static constexpr int NBUF = SingleBuf<L>::buffers;
+  // 4 lines take more than half of a CU's LDS
+  static constexpr bool kOneGroup = NBUF * 4 * LS * 8 > 80 * 1024;
+};
 template <int L, int E, bool T4>
 struct RowGeo {
   static constexpr int T = PlanOf<L, E>::T;
-  static constexpr int M = T4 ? 4 : RowShape<L, E>::M;
+  static constexpr int M = !T4 ? RowShape<L, E>::M : LineLds<L>::kOneGroup ? 2 : 4;
   static constexpr int NT = T * M;
-  __device__ static __forceinline__ int line_of(int tid) { return T4 ? ((tid >> 4) & 3) : tid / T; }
+  __device__ static __forceinline__ int line_of(int tid) { return T4 ? ((tid >> 4) & (M - 1)) : tid / T; }
   __device__ static __forceinline__ int pos_of(int tid) {
-    return T4 ? (((tid >> 6) << 4) | (tid & 15)) : tid - (tid / T) * T;
+    return T4 ? ((tid / (16 * M)) << 4) | (tid & 15) : tid - (tid / T) * T;
   }
 };
-// the tiled row kernels need T % 16 == 0, 4 T <= 1024 threads and two LDS
-// buffers of 4 lines within the 160 KiB of LDS a gfx950 work-group may use
+// the tiled row kernels need T % 16 == 0, M T <= 1024 threads and the LDS
+// buffers of M lines within the 160 KiB of LDS a gfx950 work-group may use
 template <int L, int E>
 struct T4Ok {
-  static constexpr int T = PlanOf<L, E>::T;
-  static constexpr bool value = (T % 16 == 0) && (4 * T <= 1024) && (SingleBuf<L>::buffers * LdsView<L, 4, false>::SIZE * 8 <= kLdsBytes);
+  using RG = RowGeo<L, E, true>;
+  static constexpr bool value = (RG::T % 16 == 0) && (RG::NT <= 1024) &&
+                                (SingleBuf<L>::buffers * LdsView<L, RG::M, false>::SIZE * 8 <= kLdsBytes);
 };
 
 template <int L, int E, bool DM, bool T4>
@@ -802,13 +818,13 @@ template <int L, int E>
 __global__ __launch_bounds__((RowGeo<L, E, true>::NT)) void k_row_fwd_t4(RowArgs a) {
   using RG = RowGeo<L, E, true>;
   constexpr int NR = PlanOf<L, E>::NREG;
-  using View = LdsView<L, 4, false>;
+  using View = LdsView<L, RG::M, false>;
   __shared__ float2 shA[View::SIZE];
   __shared__ float2 shB[SingleBuf<L>::value ? 1 : View::SIZE];
   const int tid = threadIdx.x;
   const int g = RG::line_of(tid), t = RG::pos_of(tid);
   const int blk = xcd_tile(blockIdx.x, gridDim.x);
-  const int line = blk * 4 + g;
+  const int line = blk * RG::M + g;
   const bool act = line < a.nlines;
   const View va{shA, g}, vb{shB, g};
   const int lc = act ? line : a.nlines - 1;
@@ -830,21 +846,25 @@ __global__ __launch_bounds__((RowGeo<L, E, true>::NT)) void k_row_fwd_t4(RowArgs
 // ---------------------------------------------------------------------------
 // Column kernels: C adjacent lines (contiguous in memory) per work-group.
 // ---------------------------------------------------------------------------
-// WIDE: at least 8 adjacent lines (64-byte segments).  In the row-major
+// kColWide: at least 8 adjacent lines (64-byte segments).  In the row-major
 // layout 32-byte segments waste much of each 128-byte line fetched, so a
 // batch with enough column groups to fill the chip runs its projection pass
 // wide; a single reconstruction keeps 4 lines per work-group and twice the
 // work-groups (the tuner times both).
-template <int L, int E, bool WIDE = false>
+// kColPairs: the tiled layout's projection pass where 4 lines leave one
+// work-group a CU (2048^2 55.0 -> 51.4 us an iteration, 4096^2 246 -> 237;
+// row-major lines keep 4: 1536^2 in batches of 7 205 -> 221).
+enum ColKind : int { kColNormal = 0, kColWide = 1, kColPairs = 2 };
+template <int L, int E, int KIND = kColNormal>
 struct ColShape {
   static constexpr int T = PlanOf<L, E>::T;
-  // C >= 4 adjacent lines (32-byte segments) and about 256 threads, within
+  // C >= Cmin adjacent lines (4: 32-byte segments) and about 256 threads, within
   // 1024 threads and the work-group's LDS
   static constexpr int LS = L + (L >> 4);
   static constexpr int Cthr = (1024 / T) >= 1 ? (1024 / T) : 1;
   static constexpr int NBUF = SingleBuf<L>::buffers;
   static constexpr int Cmem = (kLdsBytes / (NBUF * LS * 8)) >= 1 ? (kLdsBytes / (NBUF * LS * 8)) : 1;
-  static constexpr int Cmin = WIDE ? 8 : 4;
+  static constexpr int Cmin = KIND == kColWide ? 8 : KIND == kColPairs ? 2 : 4;
   // a power of two, so that column groups start on 128-byte lines (96^3 x
   // 32: 21 columns -> 16, 501 -> 479 us per iteration)
   static constexpr int pow2_floor(int v) {
@@ -859,10 +879,10 @@ struct ColShape {
   static constexpr int NT = T * C;
 };
 
-template <int L, int E, int MODE, bool WIDE = false>
-__global__ __launch_bounds__((ColShape<L, E, WIDE>::NT)) void k_col(ColArgs a) {
+template <int L, int E, int MODE, int KIND = kColNormal>
+__global__ __launch_bounds__((ColShape<L, E, KIND>::NT)) void k_col(ColArgs a) {
   using PL = PlanOf<L, E>;
-  constexpr int T = ColShape<L, E, WIDE>::T, C = ColShape<L, E, WIDE>::C, NT = ColShape<L, E, WIDE>::NT;
+  constexpr int T = ColShape<L, E, KIND>::T, C = ColShape<L, E, KIND>::C, NT = ColShape<L, E, KIND>::NT;
   constexpr int NR = PL::NREG;
   using View = LdsView<L, C, true>;
   __shared__ float2 shA[View::SIZE];
@@ -978,10 +998,10 @@ __global__ __launch_bounds__((ColShape<L, E, WIDE>::NT)) void k_col(ColArgs a) {
 // objective without amplitude margins (the branch-free projection of
 // k_col), W's cache hint a template argument (NTW 0 or 3).  Idle
 // reconstructions of a batch still leave at once.
-template <int L, int E, bool WIDE, int NTW>
-__global__ __launch_bounds__((ColShape<L, E, WIDE>::NT)) void k_col_plain(ColArgs a) {
+template <int L, int E, int KIND, int NTW>
+__global__ __launch_bounds__((ColShape<L, E, KIND>::NT)) void k_col_plain(ColArgs a) {
   using PL = PlanOf<L, E>;
-  constexpr int C = ColShape<L, E, WIDE>::C;
+  constexpr int C = ColShape<L, E, KIND>::C;
   constexpr int NR = PL::NREG;
   using View = LdsView<L, C, true>;
   __shared__ float2 shA[View::SIZE];
@@ -1106,12 +1126,13 @@ struct LengthOps {
     }
   }
   static constexpr bool t4 = T4Ok<L, E>::value;
+  static int t4_groups(int nlines) { return (nlines + RowGeo<L, E, true>::M - 1) / RowGeo<L, E, true>::M; }
   static void update(const UpdateArgs& a0, bool dm, bool tiled, hipStream_t s) {
     UpdateArgs a = a0;
     a.tw = tw();
     if (tiled) {
       if constexpr (t4) {
-        const dim3 grid((a.nlines + 3) / 4), blk(RowGeo<L, E, true>::NT);
+        const dim3 grid(t4_groups(a.nlines)), blk(RowGeo<L, E, true>::NT);
         if (dm) hipLaunchKernelGGL((k_row_update<L, E, true, true>), grid, blk, 0, s, a);
         else hipLaunchKernelGGL((k_row_update<L, E, false, true>), grid, blk, 0, s, a);
       }
@@ -1136,7 +1157,7 @@ struct LengthOps {
     const bool tab = a.alg_rec || a.beta_rec || a.rec_active;
     if (tiled) {
       if constexpr (t4) {
-        const dim3 grid((a.nlines + 3) / 4), blk(RowGeo<L, E, true>::NT);
+        const dim3 grid(t4_groups(a.nlines)), blk(RowGeo<L, E, true>::NT);
         if (tab) row_plain_launch<true, true>(a, ntw, grid, blk, s);
         else row_plain_launch<true, false>(a, ntw, grid, blk, s);
         return true;
@@ -1161,30 +1182,32 @@ struct LengthOps {
     else hipLaunchKernelGGL((k_line_project<L, E, 0>), grid, blk, 0, s, a);
     return true;
   }
-  template <bool WIDE>
+  template <int KIND>
   static bool col_plain_launch(const ColArgs& a0, hipStream_t s) {
     ColArgs a = a0;
     a.tw = tw();
     const int ntw = a.nt & 3;
     if (ntw != 0 && ntw != 3) return false;
-    const dim3 grid(((a.geo.ncontig + ColShape<L, E, WIDE>::C - 1) / ColShape<L, E, WIDE>::C) * a.geo.nouter),
-        blk(ColShape<L, E, WIDE>::NT);
-    if (ntw) hipLaunchKernelGGL((k_col_plain<L, E, WIDE, 3>), grid, blk, 0, s, a);
-    else hipLaunchKernelGGL((k_col_plain<L, E, WIDE, 0>), grid, blk, 0, s, a);
+    const dim3 grid(((a.geo.ncontig + ColShape<L, E, KIND>::C - 1) / ColShape<L, E, KIND>::C) * a.geo.nouter),
+        blk(ColShape<L, E, KIND>::NT);
+    if (ntw) hipLaunchKernelGGL((k_col_plain<L, E, KIND, 3>), grid, blk, 0, s, a);
+    else hipLaunchKernelGGL((k_col_plain<L, E, KIND, 0>), grid, blk, 0, s, a);
     return true;
   }
   static bool col_project_plain(const ColArgs& a0, bool wide, hipStream_t s) {
     if (wide) {
-      if constexpr (ColShape<L, E, true>::C > ColShape<L, E>::C) return col_plain_launch<true>(a0, s);
+      if constexpr (ColShape<L, E, kColWide>::C > ColShape<L, E>::C) return col_plain_launch<kColWide>(a0, s);
       return false;
     }
-    return col_plain_launch<false>(a0, s);
+    if constexpr (LineLds<L>::kOneGroup)
+      if (a0.geo.tshift == 2) return col_plain_launch<kColPairs>(a0, s);
+    return col_plain_launch<kColNormal>(a0, s);
   }
   static void row_t4(const RowArgs& a0, hipStream_t s) {
     if constexpr (t4) {
       RowArgs a = a0;
       a.tw = tw();
-      hipLaunchKernelGGL((k_row_fwd_t4<L, E>), dim3((a.nlines + 3) / 4), dim3(RowGeo<L, E, true>::NT), 0, s, a);
+      hipLaunchKernelGGL((k_row_fwd_t4<L, E>), dim3(t4_groups(a.nlines)), dim3(RowGeo<L, E, true>::NT), 0, s, a);
     }
   }
   static int col_blocks(const LineGeom& g) {
@@ -1204,15 +1227,15 @@ struct LengthOps {
   }
   // the projection pass with at least 8 lines per work-group, where that
   // differs from col()'s work-group
-  static constexpr bool wide = ColShape<L, E, true>::C > ColShape<L, E>::C;
+  static constexpr bool wide = ColShape<L, E, kColWide>::C > ColShape<L, E>::C;
   static int colw_blocks(const LineGeom& g) {
-    return ((g.ncontig + ColShape<L, E, true>::C - 1) / ColShape<L, E, true>::C) * g.nouter;
+    return ((g.ncontig + ColShape<L, E, kColWide>::C - 1) / ColShape<L, E, kColWide>::C) * g.nouter;
   }
   static void col_project_wide(const ColArgs& a0, hipStream_t s) {
     if constexpr (wide) {
       ColArgs a = a0;
       a.tw = tw();
-      hipLaunchKernelGGL((k_col<L, E, kColProject, true>), dim3(colw_blocks(a.geo)), dim3(ColShape<L, E, true>::NT), 0,
+      hipLaunchKernelGGL((k_col<L, E, kColProject, kColWide>), dim3(colw_blocks(a.geo)), dim3(ColShape<L, E, kColWide>::NT), 0,
                          s, a);
     }
   }
