@@ -103,7 +103,8 @@ class Engine {
   hipStream_t s = nullptr;
 
   // ---- host <-> device (rec < 0: all reconstructions, host arrays of NT) ----
-  // uploads return without waiting for the stream (upload_h2d)
+  // amplitudes, flags and tables are uploaded without waiting for the stream
+  // (upload_h2d), models with a wait
   int upload_amplitudes(const float* amp, const uint8_t* flags, int rec = -1);  // also uploads flags
   int upload_flags(const uint8_t* flags, int rec = -1);
   int download_flags(uint8_t* flags, int rec = -1);
