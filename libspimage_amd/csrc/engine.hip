@@ -9,9 +9,11 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <map>
 #include <tuple>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 namespace spx {
@@ -1890,6 +1892,7 @@ constexpr size_t kRingBytes = 64u << 20;
 
 struct UploadRing {
   std::mutex mu;
+  std::vector<hipStream_t> capturing;  // streams with a CaptureMark
   uint8_t* base = nullptr;
   size_t head = 0;
   // an event is recorded on streams of the device it was created on; the
@@ -1906,8 +1909,28 @@ struct UploadRing {
   };
   std::vector<Span> live;
   std::vector<Ev> spare;
+  bool captures(hipStream_t s) const { return std::find(capturing.begin(), capturing.end(), s) != capturing.end(); }
 };
 UploadRing g_ring;
+
+// Marks stream s as under capture.  An upload looks over the events of all
+// streams, and the query of an event last recorded on a capturing stream
+// invalidates that capture.  Events of marked streams are left alone; an
+// upload that needs their regions waits for the mark's end.
+class CaptureMark {
+ public:
+  explicit CaptureMark(hipStream_t s) : s_(s) {
+    std::lock_guard<std::mutex> lock(g_ring.mu);
+    g_ring.capturing.push_back(s);
+  }
+  ~CaptureMark() {
+    std::lock_guard<std::mutex> lock(g_ring.mu);
+    g_ring.capturing.erase(std::find(g_ring.capturing.begin(), g_ring.capturing.end(), s_));
+  }
+
+ private:
+  hipStream_t s_;
+};
 
 // Destroys the ring's events last recorded on stream s, which the caller has
 // synchronised and is about to destroy: a later query of such an event would
@@ -1946,35 +1969,45 @@ int upload_h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
   UploadRing& g = g_ring;
   int dev = 0;
   SPX_HIP(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lock(g.mu);
+  std::unique_lock<std::mutex> lock(g.mu);
   if (!g.base) SPX_HIP(hipHostMalloc((void**)&g.base, kRingBytes, hipHostMallocDefault));
   const size_t len = (bytes + 255) & ~(size_t)255;
-  size_t off = g.head;
-  if (off + len > kRingBytes) off = 0;
-  // wait for the uploads still reading [off, off + len); drop finished ones
-  for (size_t i = 0; i < g.live.size();) {
-    UploadRing::Span& sp = g.live[i];
-    const bool overlap = sp.off < off + len && off < sp.off + sp.len;
-    bool done = false;
-    if (overlap) {
-      SPX_HIP(hipEventSynchronize(sp.ev.ev));
-      done = true;
-    } else {
-      const hipError_t q = hipEventQuery(sp.ev.ev);
-      if (q != hipSuccess && q != hipErrorNotReady) SPX_HIP(q);
-      done = q == hipSuccess;
+  size_t off = 0;
+  for (bool again = true; again;) {
+    again = false;
+    off = g.head + len > kRingBytes ? 0 : g.head;
+    // wait for the uploads still reading [off, off + len); drop finished ones
+    for (size_t i = 0; i < g.live.size();) {
+      UploadRing::Span& sp = g.live[i];
+      const bool overlap = sp.off < off + len && off < sp.off + sp.len;
+      bool done = false;
+      if (g.captures(sp.ev.last)) {
+        again = again || overlap;
+      } else if (overlap) {
+        SPX_HIP(hipEventSynchronize(sp.ev.ev));
+        done = true;
+      } else {
+        const hipError_t q = hipEventQuery(sp.ev.ev);
+        if (q != hipSuccess && q != hipErrorNotReady) SPX_HIP(q);
+        done = q == hipSuccess;
+      }
+      if (done) {
+        g.spare.push_back(sp.ev);
+        sp = g.live.back();
+        g.live.pop_back();
+      } else {
+        ++i;
+      }
     }
-    if (done) {
-      g.spare.push_back(sp.ev);
-      sp = g.live.back();
-      g.live.pop_back();
-    } else {
-      ++i;
+    if (again) {  // other uploads may take the region meanwhile
+      lock.unlock();
+      std::this_thread::sleep_for(std::chrono::microseconds(20));
+      lock.lock();
     }
   }
   UploadRing::Ev ev{nullptr, dev, s};
   for (size_t i = 0; i < g.spare.size(); ++i)
-    if (g.spare[i].dev == dev) {
+    if (g.spare[i].dev == dev && !g.captures(g.spare[i].last)) {
       ev = g.spare[i];
       g.spare[i] = g.spare.back();
       g.spare.pop_back();
@@ -2429,9 +2462,14 @@ int Engine::iterate_graph(const IterParams& p, float beta, int n) {
     for (int parity = 0; parity < 2; ++parity) {
       cur = parity;
       hipGraph_t graph = nullptr;
-      SPX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      const int rc = iterate_impl(p, &beta, 1, false, nullptr);
-      const hipError_t ec = hipStreamEndCapture(s, &graph);
+      int rc = 0;
+      hipError_t ec = hipSuccess;
+      {
+        CaptureMark mark(s);
+        SPX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        rc = iterate_impl(p, &beta, 1, false, nullptr);
+        ec = hipStreamEndCapture(s, &graph);
+      }
       if (rc || ec != hipSuccess) {
         if (graph) (void)hipGraphDestroy(graph);
         cur = cur0;
