@@ -40,7 +40,7 @@ bool device_available();
 // copied with a wait); the host array may be reused at once.
 int upload_h2d(void* dst, const void* src, size_t bytes, hipStream_t s);
 // Device-to-host copy behind the work on stream s; returns when it is done
-// (up to 4 MiB through pinned blocks).
+// (up to 4 MiB into pageable memory through pinned blocks).
 int download_d2h(void* dst, const void* src, size_t bytes, hipStream_t s);
 // make_shape chooses, once per process and array shape, the plan variant
 // (elements per thread) of each axis by timing the compiled variants on the

@@ -2035,7 +2035,9 @@ int upload_h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
 // blocks (at most kDownBlocks, kept for the process): the runtime's own path
 // for small pageable arrays runs at 2.4 GB/s (1 MB 400 us, pinned 26 us; from
 // 4 MB on it pins the array and reaches 18 GB/s).  With every block in use by
-// other threads the copy goes the pageable way.
+// other threads the copy goes the pageable way.  Arrays that are page-locked
+// already need no block: 4 MiB 220 us through one, 86 us without, 1 MiB 62 and
+// 30 us.
 // ---------------------------------------------------------------------------
 namespace {
 constexpr size_t kDownBytes = 4u << 20;
@@ -2072,8 +2074,18 @@ void give_pinned(void* p) {
   g_down.spare.push_back(p);
 }
 
+// whether p points into page-locked host memory
+static bool page_locked(const void* p) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return at.type == hipMemoryTypeHost;
+}
+
 int download_d2h(void* dst, const void* src, size_t bytes, hipStream_t s) {
-  void* pin = bytes <= kDownBytes ? take_pinned() : nullptr;
+  void* pin = bytes <= kDownBytes && !page_locked(dst) ? take_pinned() : nullptr;
   const hipError_t e1 = hipMemcpyAsync(pin ? pin : dst, src, bytes, hipMemcpyDeviceToHost, s);
   const hipError_t e2 = hipStreamSynchronize(s);
   if (pin) {
