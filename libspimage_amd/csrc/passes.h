@@ -483,18 +483,19 @@ __global__ __launch_bounds__((RowShape<L, E>::NT)) void k_row(RowArgs a) {
 // whole 4 x 4 tiles (or halves, which the neighbouring work-group on the same
 // XCD completes in its L2) of the tiled one.
 //
-// 2 lines where 4 leave one work-group a CU (kOneGroup: 1215 points and more but for 2352 to 2401):
-// nothing else then loads or stores while it transforms.  Microseconds per HIO
-// iteration with 4 and with 2 lines (and the column pass's pairs, ColShape):
-// 2048^2 60.9 -> 51.4, in batches of 4 199 -> 169; 3072^2 151 -> 138; 4096^2
-// 260 (transposed) -> 237.  Shorter lines keep 4: 1024^2 with E = 8 and 2
-// lines ran 17.5 -> 16.7 us in the tuner but 14.3 -> 15.1 in a phaser.
+// 2 lines where 4 leave one work-group a CU (kOneGroup: two buffers from 1928
+// points on, one buffer from 2410): nothing else then loads or stores while it
+// transforms.  Microseconds per HIO iteration with 4 and with 2 lines (and the
+// column pass's pairs, ColShape): 2048^2 60.9 -> 51.4, in batches of 4 199 ->
+// 169; 3072^2 151 -> 138; 4096^2 260 (transposed) -> 237.  Shorter lines keep
+// 4, also where two groups do not fit a CU: their groups of 2 have too few
+// wavefronts.  1280^2 with E = 8 tiled 37.2 -> 38.9, in batches of 10 227 ->
+// 266; 1600^2 50.6 -> 59.6; 1024^2 14.3 -> 15.1.
 template <int L>
 struct LineLds {
   static constexpr int LS = L + (L >> 4);
   static constexpr int NBUF = SingleBuf<L>::buffers;
-  // 4 lines take more than half of a CU's LDS
-  static constexpr bool kOneGroup = NBUF * 4 * LS * 8 > 80 * 1024;
+  static constexpr bool kOneGroup = NBUF * 4 * LS * 8 > (NBUF == 2 ? 128 : 80) * 1024;
 };
 template <int L, int E, bool T4>
 struct RowGeo {
@@ -852,8 +853,12 @@ __global__ __launch_bounds__((RowGeo<L, E, true>::NT)) void k_row_fwd_t4(RowArgs
 // wide; a single reconstruction keeps 4 lines per work-group and twice the
 // work-groups (the tuner times both).
 // kColPairs: the tiled layout's projection pass where 4 lines leave one
-// work-group a CU (2048^2 55.0 -> 51.4 us an iteration, 4096^2 246 -> 237;
-// row-major lines keep 4: 1536^2 in batches of 7 205 -> 221).
+// work-group a CU (2048^2 55.0 -> 51.4 us an iteration, 4096^2 246 -> 237, 1024
+// columns of 4096 points 64 -> 60, of 2048 points 28.7 -> 29.7 but in batches of
+// 4 103 -> 95; row-major lines keep 4: 1536^2 in batches of 7 205 -> 221).  Not
+// by the number of groups: the compiler contracts the sums of radices 3 and 5
+// differently in the two kernels, and a reconstruction computes the same bits
+// alone and in a batch.
 enum ColKind : int { kColNormal = 0, kColWide = 1, kColPairs = 2 };
 template <int L, int E, int KIND = kColNormal>
 struct ColShape {
