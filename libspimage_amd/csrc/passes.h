@@ -690,6 +690,23 @@ __global__ __launch_bounds__((RowGeo<L, E, T4>::NT)) void k_row_update(UpdateArg
   }
 }
 
+// Wavefronts of a SIMD that the plain row pass on natural rows and the
+// transposed pass's kernel are held to (1: as the compiler decides).  With
+// these plans the compiler ends within three registers of the 128 that four
+// wavefronts may use, on either side depending on code elsewhere in the file,
+// and 129 cost the fourth.  Held, they spill 8 registers at most.
+// Microseconds per HIO iteration at 129 registers and held: 1960^2 102.7 ->
+// 90.5, 3645^2 (transposed) 360 -> 325, 1080^2 33.6 -> 32.8.  Not held: plans
+// near 168 registers (2500^2 120 with 171, 124 held to 168 by spilling 3).
+template <int L, int E>
+struct HeldWaves {
+  using PL = PlanOf<L, E>;
+  static constexpr int kept = 4 * PL::NREG + 2 * PL::NTW;  // W's and g_k's elements, twiddles
+  static constexpr int row = (PL::NREG == 6 || PL::NREG == 7) && kept >= 64 && kept <= 70 ? 4 : 1;
+  static constexpr int line =
+      PL::NREG == 9 && PL::P.maxr <= 15 && PL::NTW >= 26 && PL::NTW <= 28 && L % 7 != 0 ? 4 : 1;
+};
+
 // The real-space pass for the common case, specialised: ER / HIO / RAAR
 // without the model-before-projection output.  W's cache hint is a template
 // argument (NTW 0 or 3: loads and stores alike); the iterates' hints (nt
@@ -699,7 +716,7 @@ __global__ __launch_bounds__((RowGeo<L, E, T4>::NT)) void k_row_update(UpdateArg
 // k_row_update, without its other optional paths: kept apart, those cost
 // this pass about 0.4 us at 1024^2.
 template <int L, int E, bool T4, int NTW, bool TAB>
-__global__ __launch_bounds__((RowGeo<L, E, T4>::NT)) void k_row_plain(UpdateArgs a) {
+__global__ __launch_bounds__((RowGeo<L, E, T4>::NT), (T4 || TAB ? 1 : HeldWaves<L, E>::row)) void k_row_plain(UpdateArgs a) {
   using PL = PlanOf<L, E>;
   using RG = RowGeo<L, E, T4>;
   constexpr int M = RG::M;
@@ -1060,7 +1077,7 @@ __global__ __launch_bounds__((ColShape<L, E, KIND>::NT)) void k_col_plain(ColArg
 // belongs to reconstruction l / ncontig; idle reconstructions' lines are
 // transformed but not stored.
 template <int L, int E, int NTW>
-__global__ __launch_bounds__((RowShape<L, E>::NT)) void k_line_project(ColArgs a) {
+__global__ __launch_bounds__((RowShape<L, E>::NT), (HeldWaves<L, E>::line)) void k_line_project(ColArgs a) {
   using PL = PlanOf<L, E>;
   using RG = RowGeo<L, E, false>;
   constexpr int M = RG::M;
