@@ -517,7 +517,9 @@ static int timed_recs(int nrec, long N) {
 // timed on one reconstruction and on a batch of 16, in each layout with the
 // class's default hints, and the pair with the least cost wins, cost = the
 // slowdown against the best pair on one reconstruction + half that in the
-// batch.  (900^2: E 8 / 8 is best alone at 23.6 us and E 16 / 16 3.6 %
+// batch.  Shapes from 4 Mi pixels on are also timed with the transposed pass,
+// and alone without W's hint, as their layout will be chosen (with the
+// variants that suit that pass 3200^2 234 -> 226 us, 3840^2 318 -> 289).  (900^2: E 8 / 8 is best alone at 23.6 us and E 16 / 16 3.6 %
 // slower, but a batch of 16 takes 222 us with 8 / 8 and 163 us with 16 / 16.)
 static void choose_pair_variants(const LengthEntry* ex, const LengthEntry* ey, int ny, bool t4_shape, int* rc,
                                  int* cc) {
@@ -529,12 +531,15 @@ static void choose_pair_variants(const LengthEntry* ex, const LengthEntry* ey, i
   std::vector<float> t((size_t)2 * nvx * nvy, 1e30f);
   PairScratch b((long)nr16 * N);
   if (!b.ok) return;
+  const char* trenv = getenv("SPX_TR");
   for (int sc = 0; sc < nscale; ++sc) {
-    const int nt0 = sc == 0 ? 3 | 8 : 4 | 8;
-    for (int lay = 0; lay < 2; ++lay) {
-      if (lay == 1 && !t4_shape) continue;
+    const bool large = N >= (1L << 22);
+    const int nt0 = sc == 1 ? 4 | 8 : large ? 8 : 3 | 8;
+    for (int lay : {kLayRowMajor, kLayTiled, kLayTransposed}) {
+      if (lay == kLayTiled && !t4_shape) continue;
+      if (lay == kLayTransposed && (!large || (trenv && atoi(trenv) != 1))) continue;
       for (int r = 0; r < nvx; ++r) {
-        if (lay == 1 && !ex->var[r].t4) continue;
+        if (lay == kLayTiled && !ex->var[r].t4) continue;
         for (int c = 0; c < nvy; ++c) {
           const float ms = time_pair(b, ex->var[r], ey->var[c], nx, ny, scales[sc], lay, false, nt0);
           float& slot = t[((size_t)sc * nvx + r) * nvy + c];
