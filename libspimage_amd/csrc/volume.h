@@ -58,7 +58,7 @@ constexpr VolCfg vol_cfg(int L) {
     case 128: return {2, {8, 16, 1}, 1, {16, 1}, 2, 256, 4, 256};
     case 144: return {2, {12, 12, 1}, 2, {6, 3}, 1, 216, 4, 192};
     case 160: return {2, {10, 16, 1}, 2, {5, 4}, 1, 320, 4, 256};
-    case 192: return {2, {12, 16, 1}, 2, {6, 4}, 1, 384, 4, 384};
+    case 192: return {2, {12, 16, 1}, 2, {6, 4}, 1, 384, 4, 512};
     case 200: return {3, {8, 5, 5}, 2, {5, 5}, 1, 512, 4, 448};
     case 216: return {3, {6, 6, 6}, 2, {9, 3}, 1, 512, 4, 384};
     case 240: return {2, {15, 16, 1}, 2, {6, 5}, 1, 480, 4, 512};
