@@ -330,8 +330,9 @@ struct PairChoice {
 // layouts of a 2-D shape's Fourier-space pass
 enum PairLayout { kLayRowMajor = 0, kLayTiled = 1, kLayTransposed = 2 };
 static std::map<std::tuple<int, int, int>, PairChoice> tune_layout;
-// iterate hints chosen per 3-D shape and batch class (tune_volume_hints)
-static std::map<std::tuple<int, int, int, int>, int> volume_hints;
+// iterate hints chosen per 3-D shape, batch class and kind of passes (two or
+// per axis; tune_volume_hints)
+static std::map<std::tuple<int, int, int, int, bool>, int> volume_hints;
 
 // Tuning records.  With SPX_TUNE_FILE=<path>, every choice the tuner times
 // is appended to the file as one line of text, and the file's lines are read
@@ -340,9 +341,12 @@ static std::map<std::tuple<int, int, int, int>, int> volume_hints;
 //   shape <nx> <ny> <nz> <Ex> <Ey> <Ez>        elements per thread (0: axis of length 1)
 //   pair <nx> <ny> <class> <layout> <wide> <hints>   (layout 0 row-major, 1 tiled, 2 transposed pass)
 //   volume <nx> <ny> <nz> <class> <hints>
-// (class: batch class 0-3, hints: the non-temporal mask).  Lines that name a
-// variant this build lacks, or that do not parse, are skipped.  Caller holds
-// tune_mu.
+// (class: batch class 0-3, hints: the non-temporal mask).  Choices between
+// kernels that the first files were not timed with are named anew, so that
+// older lines for them are passed over: shape2 and pair2 of 2-D shapes with a
+// side of one_group points (two-row tiles), volume2 of two-pass volumes.  Lines
+// that name a variant this build lacks, or that do not parse, are skipped.
+// Caller holds tune_mu.
 static const char* tune_file() {
   const char* p = getenv("SPX_TUNE_FILE");
   return (p && *p) ? p : nullptr;
@@ -363,6 +367,11 @@ static int elements_of(int L, int v) {
   return e && v >= 0 && v < e->nvar ? e->var[v].E : 0;
 }
 
+// whether a shape's variants and layout are recorded as shape2 and pair2
+static bool two_row_shape(int nx, int ny, int nz) {
+  return nx > 1 && ny > 1 && nz == 1 && (one_group(nx) || one_group(ny));
+}
+
 static void load_tune_file() {
   static bool loaded = false;
   if (loaded) return;
@@ -372,20 +381,24 @@ static void load_tune_file() {
   if (!f) return;
   char line[256];
   while (fgets(line, sizeof line, f)) {
+    char kind[16];
     int a[6];
-    if (sscanf(line, "shape %d %d %d %d %d %d", &a[0], &a[1], &a[2], &a[3], &a[4], &a[5]) == 6) {
+    const int n = sscanf(line, "%15s %d %d %d %d %d %d", kind, &a[0], &a[1], &a[2], &a[3], &a[4], &a[5]) - 1;
+    const auto is = [&](const char* name, int values) { return n >= values && !strcmp(kind, name); };
+    if (is("shape", 6) || is("shape2", 6)) {
       ShapeVariants sv{};
-      bool ok = a[0] >= 1 && a[1] >= 1 && a[2] >= 1;
+      bool ok = a[0] >= 1 && a[1] >= 1 && a[2] >= 1 && is("shape2", 6) == two_row_shape(a[0], a[1], a[2]);
       for (int k = 0; ok && k < 3; ++k) {
         sv.v[k] = variant_of(a[k], a[3 + k]);
         ok = sv.v[k] >= 0;
       }
       if (ok) shape_variants[std::make_tuple(a[0], a[1], a[2])] = sv;
-    } else if (sscanf(line, "pair %d %d %d %d %d %d", &a[0], &a[1], &a[2], &a[3], &a[4], &a[5]) == 6) {
-      tune_layout[std::make_tuple(a[0], a[1], a[2])] =
-          PairChoice{a[3] == kLayTiled, a[4] != 0, a[5] & 15, a[3] == kLayTransposed};
-    } else if (sscanf(line, "volume %d %d %d %d %d", &a[0], &a[1], &a[2], &a[3], &a[4]) == 5) {
-      volume_hints[std::make_tuple(a[0], a[1], a[2], a[3])] = a[4] & 15;
+    } else if (is("pair", 6) || is("pair2", 6)) {
+      if (is("pair2", 6) == two_row_shape(a[0], a[1], 1))
+        tune_layout[std::make_tuple(a[0], a[1], a[2])] =
+            PairChoice{a[3] == kLayTiled, a[4] != 0, a[5] & 15, a[3] == kLayTransposed};
+    } else if (is("volume", 5) || is("volume2", 5)) {
+      volume_hints[std::make_tuple(a[0], a[1], a[2], a[3], is("volume2", 5))] = a[4] & 15;
     }
   }
   fclose(f);
@@ -404,8 +417,8 @@ static void record_tune_line(const char* fmt, ...) {
 }
 
 static void record_shape(int nx, int ny, int nz, const ShapeVariants& sv) {
-  record_tune_line("shape %d %d %d %d %d %d\n", nx, ny, nz, elements_of(nx, sv.v[0]), elements_of(ny, sv.v[1]),
-                   elements_of(nz, sv.v[2]));
+  record_tune_line("%s %d %d %d %d %d %d\n", two_row_shape(nx, ny, nz) ? "shape2" : "shape", nx, ny, nz,
+                   elements_of(nx, sv.v[0]), elements_of(ny, sv.v[1]), elements_of(nz, sv.v[2]));
 }
 
 static int batch_class(int nrec) { return nrec <= 1 ? 0 : nrec < 4 ? 1 : nrec < 8 ? 2 : 3; }
@@ -645,7 +658,8 @@ static int tune_pair(const LengthEntry* ex, const LengthEntry* ey, int ny, int n
     }
   }
   tune_layout[key] = PairChoice{blay == kLayTiled, bwide, bnt, blay == kLayTransposed};
-  record_tune_line("pair %d %d %d %d %d %d\n", nx, ny, batch_class(nrec), blay, bwide ? 1 : 0, bnt);
+  record_tune_line("%s %d %d %d %d %d %d\n", two_row_shape(nx, ny, 1) ? "pair2" : "pair", nx, ny, batch_class(nrec), blay,
+                   bwide ? 1 : 0, bnt);
   if (getenv("SPX_TUNE_LOG"))
     fprintf(stderr, "tune %d x %d (x%d) chose %s%s, hints %d: row E=%d col E=%d\n", nx, ny, nr,
             blay == kLayTiled ? "tiled" : blay == kLayTransposed ? "transposed" : "row-major", bwide ? " wide" : "",
@@ -1569,7 +1583,8 @@ static void enqueue_fourier(const Shape& sh, int mode, const float2* in, float2*
 static int tune_volume_hints(const Shape& sh0) {
   const char* ntenv = getenv("SPX_NT");
   if (ntenv) return atoi(ntenv) & 12;
-  const auto key = std::make_tuple(sh0.nx, sh0.ny, sh0.nz, batch_class(sh0.nrec));
+  const bool two_pass = sh0.volr != nullptr;
+  const auto key = std::make_tuple(sh0.nx, sh0.ny, sh0.nz, batch_class(sh0.nrec), two_pass);
   auto it = volume_hints.find(key);
   if (it != volume_hints.end()) return it->second;
   if (tuning_off()) return volume_hints[key] = 0;
@@ -1632,7 +1647,8 @@ static int tune_volume_hints(const Shape& sh0) {
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   if (s) (void)hipStreamDestroy(s);
-  record_tune_line("volume %d %d %d %d %d\n", sh0.nx, sh0.ny, sh0.nz, batch_class(sh0.nrec), best_mask);
+  record_tune_line("%s %d %d %d %d %d\n", two_pass ? "volume2" : "volume", sh0.nx, sh0.ny, sh0.nz, batch_class(sh0.nrec),
+                   best_mask);
   return volume_hints[key] = best_mask;
 }
 

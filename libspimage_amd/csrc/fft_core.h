@@ -554,10 +554,10 @@ constexpr int kLdsBytes = 156 * 1024;
 // buffer: a stage loads all its inputs, synchronises, then stores (two
 // barriers per stage instead of one), which halves the LDS and keeps 4 lines
 // per work-group for the column passes and the tiled layout.
+constexpr bool single_buf(int L) { return 2 * 4 * (L + (L >> 4) + 1) * 8 > kLdsBytes; }
 template <int L>
 struct SingleBuf {
-  static constexpr int LS = L + (L >> 4);
-  static constexpr bool value = 2 * 4 * (LS + 1) * 8 > kLdsBytes;
+  static constexpr bool value = single_buf(L);
   static constexpr int buffers = value ? 1 : 2;
 };
 

@@ -491,11 +491,13 @@ __global__ __launch_bounds__((RowShape<L, E>::NT)) void k_row(RowArgs a) {
 // 4, also where two groups do not fit a CU: their groups of 2 have too few
 // wavefronts.  1280^2 with E = 8 tiled 37.2 -> 38.9, in batches of 10 227 ->
 // 266; 1600^2 50.6 -> 59.6; 1024^2 14.3 -> 15.1.
+constexpr bool one_group(int L) {
+  const int LS = L + (L >> 4), nbuf = single_buf(L) ? 1 : 2;
+  return nbuf * 4 * LS * 8 > (nbuf == 2 ? 128 : 80) * 1024;
+}
 template <int L>
 struct LineLds {
-  static constexpr int LS = L + (L >> 4);
-  static constexpr int NBUF = SingleBuf<L>::buffers;
-  static constexpr bool kOneGroup = NBUF * 4 * LS * 8 > (NBUF == 2 ? 128 : 80) * 1024;
+  static constexpr bool kOneGroup = one_group(L);
 };
 template <int L, int E, bool T4>
 struct RowGeo {
