@@ -1,4 +1,5 @@
-// Column passes of lines of any length (anylen.h).
+// Column passes of lines of any length (anylen.h), of one reconstruction:
+// rec_active is not read, W of an idle slot would be projected in place.
 #include "anylen.h"
 
 namespace spx {

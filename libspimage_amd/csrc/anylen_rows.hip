@@ -53,7 +53,8 @@ __global__ __launch_bounds__((RowShape<M, E>::NT)) void k_any_row(RowArgs a, Any
 
 // The fused real-space pass: inverse x-transform, update and constraints,
 // the new iterate stored, forward x-transform (k_row_update's arithmetic for
-// one reconstruction).
+// one reconstruction: no alg_rec, beta_rec or rec_active, so batches refuse
+// these shapes).
 template <int M, int E, bool DM>
 __global__ __launch_bounds__((RowShape<M, E>::NT)) void k_any_update(UpdateArgs a, AnyLine c) {
   constexpr int T = RowShape<M, E>::T, G = RowShape<M, E>::M;

@@ -116,8 +116,9 @@ int support_update(SpxBatch* b) {
 extern "C" {
 
 SpxBatch* spx_batch_create(int nx, int ny, int nz, int nrec) {
-  // batches run the fused passes only: an axis without a Stockham plan
-  // (Bluestein transforms) is refused for any number of reconstructions
+  // an axis without a Stockham plan is refused for any number of
+  // reconstructions: the any-length passes (k_any_col, k_any_update) read no
+  // per-reconstruction tables and no activity states
   const int dims[3] = {nx, ny, nz};
   for (int d : dims)
     if (d > 1 && !spx::find_length(d)) {

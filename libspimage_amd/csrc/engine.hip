@@ -120,7 +120,7 @@ static std::mutex tune_mu;
 // Variant choices are made per array shape (nx, ny, nz), once: the first
 // engine, batch or transform of that shape tunes them and every later one
 // of the same shape, whatever its number of reconstructions or layout, uses
-// the same variants, so a reconstruction computes the same bits alone and in
+// the same variants, so that a reconstruction computes the same alone and in
 // a batch.  Shapes do not share choices: a 2-D 256 x 256 request and a
 // 256^3 volume each get the variants that suit their own passes.
 struct ShapeVariants {
@@ -305,7 +305,10 @@ static int tune_length(const LengthEntry* e, int lines, const LineGeom* col_geo)
 // size (1, 2-3, 4-7, 8 or more reconstructions: in a batch whole
 // reconstructions stay on one XCD, which favours the tiled layout, and more
 // of them fill the chip with wider work-groups).  Layouts and work-group
-// widths compute the same bits, so these choices never change a result.
+// widths run the same arithmetic in the same order and at most sizes give the
+// same bits; at some lengths with radix-3 or -5 stages (rows of 2560 or 3072
+// points, say) the compiler fuses other products in one layout's kernels, and
+// results differ in the last bits.
 // Returns true for the tiled layout.  *wide: in the row-major layout, the
 // projection pass runs with the wider work-groups
 // (LengthOps::col_project_wide), also timed here with the chosen variants;
@@ -525,7 +528,7 @@ static int timed_recs(int nrec, long N) {
 }
 
 // The variants of a 2-D shape serve every later use of the shape, alone
-// and in batches of any size (so a reconstruction computes the same bits
+// and in batches of any size (so that a reconstruction computes the same
 // either way), so they are chosen for both: each pair (row E, column E) is
 // timed on one reconstruction and on a batch of 16, in each layout with the
 // class's default hints, and the pair with the least cost wins, cost = the

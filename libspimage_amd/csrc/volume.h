@@ -15,12 +15,16 @@
 //     projection, and back.
 //
 // Both passes read and write W in place, 53 bytes a voxel in two launches
-// instead of four (the difference map: 89 instead of 154).  HBM bounds them
-// at 256^3 (a large copy moves 4.7 TB/s, so 188 us for an ER iteration), the
-// Infinity Cache and the arithmetic (100 instructions a voxel and pass)
-// below.  Microseconds per iteration before and after: 256^3 DM 489 -> 380,
-// ER 244 -> 180; 240^3 HIO 270 -> 174; 192^3 114 -> 88; 144^3 39 -> 30; 120^3
-// 40 -> 19; 64^3 13.6 -> 7; 96^3 x 8 mixed 112 -> 76; 128^3 x 3 90 -> 65.
+// instead of four (the difference map: 89 instead of 154; counted at 256^3
+// 53.7 and 107.9, as the difference map's row kernel spills 31 registers).
+// HBM bounds them at 256^3 (a large copy moves 4.7 TB/s, so 190 us for an ER
+// iteration beyond the Infinity Cache), the Infinity Cache and the arithmetic
+// (100 instructions a voxel and pass) below.  Microseconds per HIO iteration of
+// one reconstruction before and after: 64^3 14.0 -> 12.7, 80^3 20.1 both, 96^3
+// 26.2 -> 25.6, 120^3 61 -> 32, 128^3 45 -> 31, 144^3 52 -> 46, 160^3 80 -> 70,
+// 192^3 106 -> 97, 200^3 124 -> 106, 216^3 190 -> 165, 240^3 238 -> 180, 256^3
+// 214 -> 174; difference map 64^3 26.6 -> 18.2, 128^3 88 -> 56, 256^3 465 ->
+// 411; batches of 8 96^3 113 -> 78, 128^3 226 -> 161.
 //
 // The split: tiles of 64 KiB and less, so that two or more work-groups share
 // a CU and one loads while another transforms.  At 256^3 the row tile is 32 x
@@ -30,8 +34,9 @@
 // with C = 2 2.2 TB/s).  Up to 128 the column tiles are also 4 wide: 96^3 x 8
 // 49 us a pass with C = 8 (two work-groups of 56 KiB a CU), 32 us with 4.
 //
-// Instances exist for the lengths of vol_cfg (multiples of 8 up to 256): the
-// row pass for nx = ny = L, the column pass for nz = L.
+// Instances exist for the lengths of vol_cfg (multiples of 8 from 64 to 256
+// without a factor 7): the row pass for nx = ny = L, the column pass for nz = L.
+// Other volumes, all with ny != nx among them, keep the passes per axis.
 #pragma once
 #include "passes.h"
 
@@ -47,7 +52,8 @@ struct VolCfg {
 };
 
 // Work-group sizes keep the butterflies of the widest stages at a whole
-// number per thread, about 16 elements each.
+// number per thread, about 16 elements each (192: 512 threads for the column
+// tile's 512 radix-12 butterflies; 192^3 HIO took 115 us with 384, 97 now).
 constexpr VolCfg vol_cfg(int L) {
   switch (L) {
     case 64: return {2, {8, 8, 1}, 1, {8, 1}, 4, 256, 4, 256};
@@ -200,6 +206,8 @@ struct VolRow {
   static constexpr int NY = RB * (A / YL) * L;            // its butterflies
   static constexpr int IY = per_thread<NY, NT>;
   static_assert(IY * YL <= 32, "the support bits of a thread fit a word");
+  // the radix-16 rows of 128 need 166 registers: held to the 128 of a fourth
+  // wave they spill (128^3 HIO 31.5 -> 38.8 us, batches of 8 161 -> 245)
   static constexpr int WPE = L == 128 ? 3 : waves_per_simd((NBUF * SIZE + vol_table_size(L)) * 8, NT);
 };
 
