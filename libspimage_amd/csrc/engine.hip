@@ -706,12 +706,44 @@ struct FourierLayout {
 
 // amplitudes as the projection reads them: unmeasured pixels get the NaN
 // pattern kUnmeasuredBits, measured NaNs the canonical quiet NaN
+__device__ __forceinline__ float encoded_amp(float a, uint8_t flag) {
+  if (!(flag & kMeasured)) return __uint_as_float(kUnmeasuredBits);
+  return isnan(a) ? __uint_as_float(0x7FC00000u) : a;
+}
+
 __global__ void k_encode_amp(const float* amp, const uint8_t* flags, float* ampx, long n, FourierLayout at) {
-  GRID_STRIDE(i, n) {
-    float a = amp[i];
-    if (!(flags[i] & kMeasured)) a = __uint_as_float(kUnmeasuredBits);
-    else if (isnan(a)) a = __uint_as_float(0x7FC00000u);
-    ampx[at(i)] = a;
+  GRID_STRIDE(i, n) ampx[at(i)] = encoded_amp(amp[i], flags[i]);
+}
+
+// The same for two-pass volumes, a tile of 32 x by 32 z of one y through LDS:
+// rows are read 128 bytes at a time and the column pass's order is written in
+// runs of 32 C values (k_encode_amp's stores of C values each wrote 8 to 9 bytes
+// a voxel instead of 4: 96^3 x 8 32 -> 15 us, one of them 9.7 -> 8.6, 256^3 99 ->
+// 60).  Grid (tiles of x times tiles of z, ny, reconstructions).
+template <int C>
+__global__ __launch_bounds__(256) void k_encode_amp_vol(const float* amp, const uint8_t* flags, float* ampx, int nx,
+                                                        int ny, int nz) {
+  constexpr int TILE = 32, PER = TILE * TILE / 256;
+  __shared__ float tile[TILE][TILE + 1];
+  const int tid = threadIdx.x, tilesx = (nx + TILE - 1) / TILE;
+  const int z0 = blockIdx.x / tilesx * TILE, x0 = blockIdx.x % tilesx * TILE, y = blockIdx.y;
+  const long base = (long)blockIdx.z * nx * ny * nz;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int x = tid % TILE, z = tid / TILE + k * (256 / TILE);
+    if (x0 + x < nx && z0 + z < nz) {
+      const long i = base + ((long)(z0 + z) * ny + y) * nx + x0 + x;
+      tile[z][x] = encoded_amp(amp[i], flags[i]);
+    }
+  }
+  __syncthreads();
+  // vol_amp_index of x0, y, z0; groups of C columns lie kVolB nz C apart
+  const int A = ny / kVolB, d = y / A, c = y - d * A;
+  float* out = ampx + base + (((long)(c * (nx / C) + x0 / C) * kVolB + d) * nz + z0) * C;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int e = tid + k * 256, z = e / C % TILE, g = e / (TILE * C), x = g * C + e % C;
+    if (x0 + x < nx && z0 + z < nz) out[(long)g * kVolB * nz * C + e % (TILE * C)] = tile[z][x];
   }
 }
 
@@ -1310,6 +1342,18 @@ static FourierLayout layout_of(const Shape& sh) {
   return FourierLayout{sh.nx, sh.ny, sh.nz, sh.t4 ? 1 : 0, sh.volc ? sh.volc->C : 0};
 }
 
+// nrec reconstructions' amplitudes into the Fourier-space layout
+static void enqueue_encode_amp(const Shape& sh, int nrec, const float* amp, const uint8_t* flags, float* ampx,
+                               hipStream_t s) {
+  if (sh.volc && sh.volc->C == 4) {
+    const dim3 grid((sh.nx + 31) / 32 * ((sh.nz + 31) / 32), sh.ny, nrec);
+    hipLaunchKernelGGL(k_encode_amp_vol<4>, grid, dim3(256), 0, s, amp, flags, ampx, sh.nx, sh.ny, sh.nz);
+  } else {
+    const long n = (long)sh.nx * sh.ny * sh.nz * nrec;
+    hipLaunchKernelGGL(k_encode_amp, ew_grid(n), dim3(256), 0, s, amp, flags, ampx, n, layout_of(sh));
+  }
+}
+
 // ---------------------------------------------------------------------------
 // two-pass volumes (volume.h)
 // ---------------------------------------------------------------------------
@@ -1872,7 +1916,7 @@ int Engine::alloc_all() {
   SPX_HIP(hipMemsetAsync(flags, 0, (size_t)NT, s));
   SPX_HIP(hipMemsetAsync(absb, 0, f, s));
   SPX_HIP(hipMemsetAsync(ctl, 0, sizeof(unsigned) * (size_t)kCtlStride * nrec, s));
-  hipLaunchKernelGGL(k_encode_amp, ew_grid(NT), dim3(256), 0, s, absb, flags, ampx, NT, layout_of(sh));
+  enqueue_encode_amp(sh, nrec, absb, flags, ampx, s);
   // no wait: everything later on the stream is ordered behind these
   SPX_HIP(hipGetLastError());
   return 0;
@@ -2126,8 +2170,7 @@ int Engine::upload_amplitudes(const float* amp, const uint8_t* fl, int rec) {
   const long off = rec < 0 ? 0 : rec * N, n = rec < 0 ? NT : N;
   if (int rc = upload_h2d(absb + off, amp, sizeof(float) * n, s)) return rc;
   if (int rc = upload_h2d(flags + off, fl, (size_t)n, s)) return rc;
-  hipLaunchKernelGGL(k_encode_amp, ew_grid(n), dim3(256), 0, s, absb + off, flags + off, ampx + off, n,
-                     layout_of(sh));
+  enqueue_encode_amp(sh, rec < 0 ? nrec : 1, absb + off, flags + off, ampx + off, s);
   SPX_HIP(hipGetLastError());
   ++flags_version;
   ++amp_version;
